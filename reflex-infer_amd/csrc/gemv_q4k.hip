@@ -695,9 +695,11 @@ __global__ __launch_bounds__(256) void gemv_lds_kernel(GemvParams p) {
     const int wave = blockIdx.x * 4 + wv;
     const bool active = wave < p.total_units;
     const Range rg = range_of_unit(p, active ? wave : 0);
-    const int r0 = (wave - rg.first_unit) * p.per_unit;
-    const int r1 = active ? min(r0 + p.per_unit, rg.rows) : r0;
-    const int n_items = (r1 > r0 ? r1 - r0 : 0) * J;
+    // inactive waves (the last workgroup's, when the units are not a multiple
+    // of four) take no rows of range 0: their clamped loads read its row 0
+    const int r0 = active ? (wave - rg.first_unit) * p.per_unit : 0;
+    const int r1 = active ? min(r0 + p.per_unit, rg.rows) : 0;
+    const int n_items = (r1 - r0) * J;
     const uint32_t row_bytes = (uint32_t)p.nb * kBlockBytes;
 
     // Items are walked in order by two cursors (loads run up to two batches
