@@ -23,7 +23,7 @@
  *     work; no entry point but rxq4_release_workspace synchronises the
  *     device or the stream.  The one allocation is the fp32 workspace of the
  *     split launches (split-K GEMM with few output tiles, small-batch
- *     products on long rows, decode attention over long sequences): 48 MiB
+ *     products on long rows, attention over long cached contexts): 48 MiB
  *     per (device, stream), made by the first such launch on that stream,
  *     never resized, and kept until rxq4_release_workspace(stream) frees it,
  *     so a HIP graph captured on a stream stays valid whatever runs later,

@@ -460,12 +460,11 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnParams p) {
 //                   keep ~22 bits of the fp32 probabilities.
 // Causal: query row (t, h) sees positions [0, start + t]; rows of a tile
 // past that get probability 0 (rows with nothing visible yet keep m = -inf).
-// Launch bounds: two resident workgroups of the one-group form per CU (LDS
-// allows two), which caps a wave at 256 registers; uncapped, the compiler
-// spread the one-group kernel over AGPRs with ~320 accvgpr moves per two
-// tiles (2048 tokens 129 -> 119 us with the cap).
-template <int HD, int HB, bool I8, int G>
-__global__ __launch_bounds__(256 * G, 2 / G) void attn_prefill_mfma(AttnParams p, int start, int n_tok) {
+// This kernel serves prompts of at most one workgroup per CU and few tiles (see
+// rows16_preferred); attn_prefill.hip the rest.
+template <int HD, int HB, bool I8>
+__global__ __launch_bounds__(512) void attn_prefill_mfma(AttnParams p, int start, int n_tok) {
+    constexpr int G = 2;               // wave groups
     constexpr int TPW = 16 / HB;       // tokens per wave
     constexpr int TPB = 4 * TPW;       // tokens per workgroup
     // V is stored row-major with 16-byte writes and read transposed
@@ -482,7 +481,7 @@ __global__ __launch_bounds__(256 * G, 2 / G) void attn_prefill_mfma(AttnParams p
     __shared__ float kscg[G][2][kAttnTile], vscg[G][2][kAttnTile];
     static_assert(2 * kAttnTile * KROW * 2 >= 256 * (HD / 4 + 2) * 4, "merge buffer fits");
 
-    const int q = G == 1 ? 0 : threadIdx.x >> 8;  // group: KV tiles G*j + q
+    const int q = threadIdx.x >> 8;  // group: KV tiles G*j + q
     const int tid = threadIdx.x & 255, lane = tid & 63, w = tid >> 6;
     uint16_t (*kt)[kAttnTile * KROW] = ktg[q];
     uint16_t (*vt)[VSZ] = vtg[q];
@@ -746,7 +745,7 @@ __global__ __launch_bounds__(256 * G, 2 / G) void attn_prefill_mfma(AttnParams p
     // its own with the usual rescaling (scores are in log2 units).
     float *mb = reinterpret_cast<float *>(&ktg[G - 1][0][0]);
     constexpr int NO = HD / 4;  // O values per thread
-    if (G == 2 && q == 1) {
+    if (q == 1) {
 #pragma unroll
         for (int dt = 0; dt < HD / 16; ++dt)
 #pragma unroll
@@ -754,9 +753,9 @@ __global__ __launch_bounds__(256 * G, 2 / G) void attn_prefill_mfma(AttnParams p
         mb[NO * 256 + tid] = m;
         mb[(NO + 1) * 256 + tid] = l;
     }
-    if (G == 2) lds_sync();
+    lds_sync();
     if (q == 1) return;
-    if (G == 2) {
+    {
         const float m1 = mb[NO * 256 + tid], l1 = mb[(NO + 1) * 256 + tid];
         const float mm = fmaxf(m, m1);
         const bool live = mm != -INFINITY;
@@ -1015,33 +1014,44 @@ __global__ __launch_bounds__(256, 2) void attn_decode_mfma(AttnParams p) {
     }
 }
 
-template <int HD, bool I8, int G>
-static void launch_prefill_g(unsigned grid, int hb, const AttnParams &p, int start, int n_tok,
-                             hipStream_t st) {
-    switch (hb) {
-        case 1: attn_prefill_mfma<HD, 1, I8, G><<<grid, 256 * G, 0, st>>>(p, start, n_tok); break;
-        case 2: attn_prefill_mfma<HD, 2, I8, G><<<grid, 256 * G, 0, st>>>(p, start, n_tok); break;
-        case 4: attn_prefill_mfma<HD, 4, I8, G><<<grid, 256 * G, 0, st>>>(p, start, n_tok); break;
-        case 8: attn_prefill_mfma<HD, 8, I8, G><<<grid, 256 * G, 0, st>>>(p, start, n_tok); break;
-        default: attn_prefill_mfma<HD, 16, I8, G><<<grid, 256 * G, 0, st>>>(p, start, n_tok); break;
-    }
+// HB = the largest power of two <= 16 dividing the GQA group, and the
+// workgroups of attn_prefill_mfma.
+static int rows16_heads(int group) {
+    int hb = 1;
+    while (hb < 16 && group % (2 * hb) == 0) hb *= 2;
+    return hb;
+}
+static int64_t rows16_grid(int n_kv, int group, int n_tok) {
+    const int hb = rows16_heads(group), tpb = 4 * (16 / hb);
+    return (int64_t)n_kv * (group / hb) * (((int64_t)n_tok + tpb - 1) / tpb);
 }
 
-// Two wave groups per workgroup (KV tiles split between them) while the
-// query rows give at most one wave per SIMD; more rows fill the SIMDs with
-// one group and keep the LDS of two workgroups per CU (512 tokens x 32
-// heads: 18.9 -> 17.1 us with two groups; 2048 tokens: 138.6 us with one,
-// 145.0 with two).
+// Whether attn_prefill_mfma (64 query rows a workgroup, never split) is the
+// faster one: with one round of workgroups it takes 5.0 + 1.08 us a tile at
+// head_dim 128 (3.8 + 0.78 at 64), its shorter chain against the 128-row
+// kernel's reuse and splits.  Measured, 32 / 8 heads of 128, this kernel
+// against the other: 8 tokens 6.4 / 7.2 us, 200 9.9 / 11.2, 512 14.7 / 17.5;
+// past one round 640 tokens 21.2 / 19.7, 1000 34.7 / 29, 2048 104 / 68; after
+// cached positions 45 + 400 12.5 / 13.4, 45 + 800 19.4 / 14.7, 45 + 8000
+// 134 / 27.
+static bool rows16_preferred(int n_heads, int n_kv, int head_dim, int n_tok, int start, int cus) {
+    if (head_dim != 64 && head_dim != 128) return false;
+    if (rows16_grid(n_kv, n_heads / n_kv, n_tok) > cus) return false;
+    const int tiles = (start + n_tok + kAttnTile - 1) / kAttnTile;
+    const double us = head_dim == 64 ? 3.8 + 0.78 * tiles : 5.0 + 1.08 * tiles;
+    return us <= prefill_attention_us(n_heads, n_kv, head_dim, n_tok, start);
+}
+
 template <int HD, bool I8>
-static void launch_prefill_hd(const AttnParams &p, int hb, int start, int n_tok, hipStream_t st) {
-    const int units = p.n_kv * (p.group / hb);
-    const int tpb = 4 * (16 / hb);
-    const unsigned grid = (unsigned)(units * ((n_tok + tpb - 1) / tpb));
-    const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
-    if ((int64_t)grid * 4 <= 4 * cus)
-        launch_prefill_g<HD, I8, 2>(grid, hb, p, start, n_tok, st);
-    else
-        launch_prefill_g<HD, I8, 1>(grid, hb, p, start, n_tok, st);
+static void launch_prefill_hd(const AttnParams &p, int start, int n_tok, hipStream_t st) {
+    const unsigned grid = (unsigned)rows16_grid(p.n_kv, p.group, n_tok);
+    switch (rows16_heads(p.group)) {
+        case 1: attn_prefill_mfma<HD, 1, I8><<<grid, 512, 0, st>>>(p, start, n_tok); break;
+        case 2: attn_prefill_mfma<HD, 2, I8><<<grid, 512, 0, st>>>(p, start, n_tok); break;
+        case 4: attn_prefill_mfma<HD, 4, I8><<<grid, 512, 0, st>>>(p, start, n_tok); break;
+        case 8: attn_prefill_mfma<HD, 8, I8><<<grid, 512, 0, st>>>(p, start, n_tok); break;
+        default: attn_prefill_mfma<HD, 16, I8><<<grid, 512, 0, st>>>(p, start, n_tok); break;
+    }
 }
 
 template <bool I8>
@@ -1062,6 +1072,15 @@ hipError_t launch_attention(uint16_t *out, const uint16_t *q, const void *k, con
                             const float *ks, const float *vs, int n_heads, int n_kv,
                             int head_dim, int n_tok, int seq0, float scale, int kv_int8,
                             hipStream_t st) {
+    const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
+    const bool rows16 = n_tok > 1 && tuning().attn_mfma &&
+                        rows16_preferred(n_heads, n_kv, head_dim, n_tok, seq0 - 1, cus);
+    if (n_tok > 1 && tuning().attn_mfma && !rows16) {
+        // callers' limit for the head sizes that had a grid row per token
+        if (head_dim != 64 && head_dim != 128 && n_tok > 65535) return hipErrorInvalidValue;
+        return launch_prefill_attention(out, q, k, v, ks, vs, n_heads, n_kv, head_dim, n_tok, seq0 - 1,
+                                        scale, kv_int8, st);
+    }
     AttnParams p{};
     p.out = out;
     p.q = q;
@@ -1089,7 +1108,6 @@ hipError_t launch_attention(uint16_t *out, const uint16_t *q, const void *k, con
     p.chunk = seq0 + n_tok;  // whole sequence
     if (n_tok == 1 && seq0 > kAttnTile) {
         // Decode: split the positions so that about 4 workgroups per CU run.
-        const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
         int cap = tuning().attn_split ? std::min(64, tuning().attn_split) : 64;
         // the chunk partials (n_heads x chunks x (head_dim + 2) fp32) must fit the workspace
         const size_t per_chunk = (size_t)n_heads * (head_dim + 2) * sizeof(float);
@@ -1108,20 +1126,13 @@ hipError_t launch_attention(uint16_t *out, const uint16_t *q, const void *k, con
             if (e != hipSuccess) return e;
         }
     }
-    if (n_tok > 1 && (head_dim == 64 || head_dim == 128) && tuning().attn_mfma) {
-        // Prefill on the matrix cores; HB = the largest power of two <= 16
-        // dividing the GQA group.
-        int hb = 1;
-        while (hb < 16 && p.group % (2 * hb) == 0) hb *= 2;
-        const int start = seq0 - 1;
-        const int64_t blocks = (int64_t)n_kv * (p.group / hb) * ((n_tok + 4 * (16 / hb) - 1) / (4 * (16 / hb)));
-        if (blocks > 0x7FFFFFFF) return hipErrorInvalidValue;
+    if (rows16) {
         if (head_dim == 64) {
-            if (kv_int8) launch_prefill_hd<64, true>(p, hb, start, n_tok, st);
-            else launch_prefill_hd<64, false>(p, hb, start, n_tok, st);
+            if (kv_int8) launch_prefill_hd<64, true>(p, seq0 - 1, n_tok, st);
+            else launch_prefill_hd<64, false>(p, seq0 - 1, n_tok, st);
         } else {
-            if (kv_int8) launch_prefill_hd<128, true>(p, hb, start, n_tok, st);
-            else launch_prefill_hd<128, false>(p, hb, start, n_tok, st);
+            if (kv_int8) launch_prefill_hd<128, true>(p, seq0 - 1, n_tok, st);
+            else launch_prefill_hd<128, false>(p, seq0 - 1, n_tok, st);
         }
         return hipGetLastError();
     }

@@ -164,6 +164,15 @@ hipError_t launch_attention(uint16_t *out, const uint16_t *q, const void *k, con
                             int head_dim, int n_tok, int seq0, float scale, int kv_int8,
                             hipStream_t stream);
 
+// The same for two or more tokens, 128 query rows a workgroup and the positions
+// split over workgroups where that pays: token t sees positions [0, start + t].
+// prefill_attention_us: its launch model's time (the dispatch's measure).
+double prefill_attention_us(int n_heads, int n_kv, int head_dim, int n_tok, int start);
+hipError_t launch_prefill_attention(uint16_t *out, const uint16_t *q, const void *k, const void *v,
+                                    const float *ks, const float *vs, int n_heads, int n_kv,
+                                    int head_dim, int n_tok, int start, float scale, int kv_int8,
+                                    hipStream_t stream);
+
 // fp32 rows -> Q4_K blocks (min/max quantiser).
 hipError_t launch_quantize(uint8_t *dst, const float *src, int64_t n_blocks,
                            hipStream_t stream);
