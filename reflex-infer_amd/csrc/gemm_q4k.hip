@@ -320,37 +320,47 @@ struct GemmFmt<14> {
     }
 };
 
-// LDS of one workgroup: the x ring, reused for the staged output tile.
-template <int TM, int NW = 8>
+// LDS of one workgroup: the x rings of its KG wave groups, reused for the
+// staged output tile (one group) or the other groups' sums.
+template <int TM, int NW = 8, int KG = 1>
 constexpr int gemm_lds_bytes() {
-    return TM * out_pitch<NW>() > kRing * TM * 128 ? TM * out_pitch<NW>() : kRing * TM * 128;
+    return KG == 1 && TM * out_pitch<NW>() > kRing * TM * 128 ? TM * out_pitch<NW>() : KG * kRing * TM * 128;
 }
 
 // One output tile of an NW-wave workgroup (NW = 8: two waves per SIMD; 4:
 // one): rows [32 * NW * row_tile, +32 * NW) x tokens [TM * tok_tile, +TM)
-// over super-blocks [split * sb_per_split, +sb_per_split).
-template <int T, int XT, int YT, int TM, int NW = 8>
+// over super-blocks [split * sb_per_split, +sb_per_split).  KG > 1: KG groups
+// of NW waves share the tile and take consecutive parts of those super-blocks,
+// each with its own x ring; group 0 adds the others' sums.
+template <int T, int XT, int YT, int TM, int NW = 8, int KG = 1>
 __device__ __forceinline__ void gemm_tile(const GemmParams &p, uint8_t *lds, int split,
                                           int row_tile, int tok_tile) {
     using F = GemmFmt<T>;
-    // TM tokens per workgroup tile (128 or 256)
+    // TM tokens per workgroup tile (32 to 256)
     constexpr int NT = TM / 32;      // 32-token fragments per wave
     constexpr int MPS = 4 * NT;      // MFMAs per stage and wave
+    constexpr int PPM = MPS < 16 ? 16 / MPS : 1;  // operand pieces behind an MFMA
+    constexpr int MPP = MPS < 16 ? 1 : MPS / 16;  // ... of every MPP-th
     constexpr int RPW = 32 * NW;     // weight rows per workgroup
     constexpr int THREADS = 64 * NW;
     constexpr int kOutPitch = out_pitch<NW>();
     constexpr int kXLoads = TM / (8 * NW); // 1 KB direct-to-LDS copies per wave per stage
     constexpr int kQLoads = F::kQLoads, kHLoads = F::kHLoads;
-    constexpr int kLook = 6;         // B fragments are read kLook MFMAs before use
+    constexpr int kLook = MPS < 6 ? MPS : 6;  // B fragments are read kLook MFMAs before use
     constexpr int kBufBytes = TM * 128;                        // one stage of x
     const int tile = row_tile * p.tok_tiles + tok_tile;
-    const int sb0 = split * p.sb_per_split;
-    const int nsb = min(p.nb, sb0 + p.sb_per_split) - sb0;
+    const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / THREADS);
+    const int split_n = min(p.nb - split * p.sb_per_split, p.sb_per_split);
+    const int part = (split_n + KG - 1) / KG;  // super-blocks a group, the last ones fewer
+    const int nsb = max(0, min(part, split_n - kg * part));
+    // (a group without super-blocks loads, and discards, the row's last one)
+    const int sb0 = min(p.nb - 1, split * p.sb_per_split + kg * part);
     const int n_stages = 4 * nsb;
 
-    const int tid = threadIdx.x;
+    const int tid = KG == 1 ? threadIdx.x : threadIdx.x - kg * THREADS;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    lds += kg * (kRing * TM * 128);
     const int lr = lane & 31;   // row (A) / token (B) within a 32-fragment
     const int h = lane >> 5;    // half of the stage's weights of the row
     const int K = p.K;
@@ -371,7 +381,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams &p, uint8_t *lds, int
     } else {
         ld.row = p.w + (int64_t)min(row_base + lr, p.M - 1) * row_bytes + sb0 * F::kBytes;
     }
-    ld.nsb = nsb;
+    ld.nsb = KG == 1 ? nsb : max(1, nsb);
     ld.h = h;
 
     // Direct-to-LDS copies of the x tile: TM / 8 chunks of 1 KB (8 tokens)
@@ -391,7 +401,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams &p, uint8_t *lds, int
     // Stage s's copies (clamped to the last stage) into ring buffer s % 4;
     // the stage's k offset is the wave-uniform soffset of the load.
     auto issue_x = [&](int buf, int s) {
-        const int k0b = (sb0 * 256 + F::stage_elem(min(s, n_stages - 1))) * 2;
+        const int k0b = (sb0 * 256 + F::stage_elem(min(s, KG == 1 ? n_stages - 1 : max(0, n_stages - 1)))) * 2;
 #pragma unroll
         for (int i = 0; i < kXLoads; ++i)
             buffer_to_lds16(xrsrc, lds + buf * kBufBytes + (wave + NW * i) * 1024, xoff[i], k0b);
@@ -443,7 +453,12 @@ __device__ __forceinline__ void gemm_tile(const GemmParams &p, uint8_t *lds, int
 #pragma unroll
     for (int n = 0; n < kLook; ++n) bq[n] = read_b(0, n);
 
-    for (int sbi = 0; sbi < nsb; ++sbi) {
+    for (int sbi = 0; sbi < part; ++sbi) {
+        if (KG > 1 && sbi >= nsb) {  // uniform: only the other groups' barriers are left
+#pragma unroll
+            for (int il = 0; il < 4; ++il) lds_barrier();
+            continue;
+        }
 #pragma unroll
         for (int il = 0; il < 4; ++il) {
             const int s = 4 * sbi + il;
@@ -479,14 +494,18 @@ __device__ __forceinline__ void gemm_tile(const GemmParams &p, uint8_t *lds, int
 #pragma unroll
             for (int n = 0; n < MPS; ++n) {
                 const int k = n / NT, tf = n % NT;
-                acc[tf] = mfma32<XT>(acur[k], bq[n & 7], acc[tf]);
-                if (n % (MPS / 16) == 0) {
-                    const int pi = n / (MPS / 16);  // piece pi & 3 of k-step pi >> 2
-                    F::template piece<XT>(pi >> 2, pi & 3, (il + 1) & 3, qn, hn, gs, pc,
-                                          anext[pi >> 2]);
+                const int seq = il * MPS + n;  // four stages are a multiple of 8 MFMAs
+                acc[tf] = mfma32<XT>(acur[k], bq[seq & 7], acc[tf]);
+                if (n % MPP == 0) {
+#pragma unroll
+                    for (int i = 0; i < PPM; ++i) {
+                        const int pi = n / MPP * PPM + i;  // piece pi & 3 of k-step pi >> 2
+                        F::template piece<XT>(pi >> 2, pi & 3, (il + 1) & 3, qn, hn, gs, pc,
+                                              anext[pi >> 2]);
+                    }
                 }
                 const int nr = n + kLook;
-                bq[nr & 7] = nr < MPS ? read_b(il, nr) : read_b((il + 1) & 3, nr - MPS);
+                bq[(seq + kLook) & 7] = nr < MPS ? read_b(il, nr) : read_b((il + 1) & 3, nr - MPS);
             }
             if (il == 3) hcur = hnext;
         }
@@ -496,6 +515,29 @@ __device__ __forceinline__ void gemm_tile(const GemmParams &p, uint8_t *lds, int
     wait_vmcnt<0>();
     wait_lgkmcnt0();
 
+    if constexpr (KG > 1) {
+        // every wave is done with the rings; groups 1.. leave their sums there
+        static_assert((KG - 1) * NT * 16 * THREADS * 4 <= KG * kRing * TM * 128, "the sums fit the rings");
+        lds_barrier();
+        f32x4 *sums = reinterpret_cast<f32x4 *>(lds - kg * (kRing * TM * 128));
+        if (kg > 0)
+#pragma unroll
+            for (int e = 0; e < 4 * NT; ++e)
+                sums[((kg - 1) * 4 * NT + e) * THREADS + tid] =
+                    f32x4{acc[e / 4][4 * (e % 4)], acc[e / 4][4 * (e % 4) + 1], acc[e / 4][4 * (e % 4) + 2],
+                          acc[e / 4][4 * (e % 4) + 3]};
+        wait_lgkmcnt0();
+        lds_barrier();
+        if (kg > 0) return;
+#pragma unroll
+        for (int g = 1; g < KG; ++g)
+#pragma unroll
+            for (int e = 0; e < 4 * NT; ++e) {
+                const f32x4 v = sums[((g - 1) * 4 * NT + e) * THREADS + tid];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[e / 4][4 * (e % 4) + i] += v[i];
+            }
+    }
     if (p.splits > 1) {
         // partial tile: per thread NT x 4 float4 in (tf, j) order
         f32x4 *part = reinterpret_cast<f32x4 *>(p.ws) +
@@ -508,7 +550,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams &p, uint8_t *lds, int
                                                  acc[tf][4 * j + 2], acc[tf][4 * j + 3]};
         return;
     }
-    if (YT != RXQ4_DTYPE_F32 && (p.M & 7) == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0) {
+    if (KG == 1 && YT != RXQ4_DTYPE_F32 && (p.M & 7) == 0 && (reinterpret_cast<uintptr_t>(p.y) & 15) == 0) {
         // Stage the tile as [token][RPW rows] (16-bit) in the ring, then
         // write 16 bytes per lane: RPW / 8 lanes cover one token's rows.
         lds_barrier();  // every wave is done reading the ring
@@ -563,9 +605,9 @@ __device__ __forceinline__ void gemm_tile(const GemmParams &p, uint8_t *lds, int
         }
 }
 
-template <int T, int XT, int YT, int TM, int NW = 8>
-__global__ __launch_bounds__(64 * NW) void gemm_kernel(GemmParams p) {
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[gemm_lds_bytes<TM, NW>()];
+template <int T, int XT, int YT, int TM, int NW = 8, int KG = 1>
+__global__ __launch_bounds__(64 * NW * KG) void gemm_kernel(GemmParams p) {
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[gemm_lds_bytes<TM, NW, KG>()];
     const int L = blockIdx.x;
     const int V = (L % 8) * p.units_per_xcd + L / 8;  // consecutive units share an XCD
     if (V >= p.total_units) return;
@@ -589,7 +631,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_kernel(GemmParams p) {
         row_tile = t / p.tok_tiles;
         tok_tile = t % p.tok_tiles;
     }
-    gemm_tile<T, XT, YT, TM, NW>(p, lds, split, row_tile, tok_tile);
+    gemm_tile<T, XT, YT, TM, NW, KG>(p, lds, split, row_tile, tok_tile);
 }
 
 // Mixed token tiles for GEMMs that fill the CUs between one and two times
@@ -974,7 +1016,18 @@ __global__ __launch_bounds__(256) void tokens_reduce_kernel(void *__restrict__ y
     store_out<YT>(y, i, s);
 }
 
-template <int T, int XT, int YT, int TM, int NW = 8>
+hipError_t launch_tokens_reduce(void *y, int y_dtype, const float *ws, int64_t n, int splits,
+                                hipStream_t st) {
+    const unsigned g = (unsigned)((n + 255) / 256);
+    switch (y_dtype) {
+        case RXQ4_DTYPE_F32: tokens_reduce_kernel<RXQ4_DTYPE_F32><<<g, 256, 0, st>>>(y, ws, n, splits); break;
+        case RXQ4_DTYPE_BF16: tokens_reduce_kernel<RXQ4_DTYPE_BF16><<<g, 256, 0, st>>>(y, ws, n, splits); break;
+        default: tokens_reduce_kernel<RXQ4_DTYPE_F16><<<g, 256, 0, st>>>(y, ws, n, splits); break;
+    }
+    return hipGetLastError();
+}
+
+template <int T, int XT, int YT, int TM, int NW = 8, int KG = 1>
 static hipError_t launch_gemm_t(void *y, const uint8_t *w, const uint16_t *x, int M, int N,
                                 int K, hipStream_t st, const Scratch &sc) {
     constexpr int RPW = 32 * NW, THREADS = 64 * NW;
@@ -996,9 +1049,10 @@ static hipError_t launch_gemm_t(void *y, const uint8_t *w, const uint16_t *x, in
     const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
     // Split K into as many parts as keep every unit resident at once (one
     // workgroup per CU: tiles * splits <= CUs), at least 2 super-blocks a
-    // split: 32 tiles on 256 CUs split 8, 86 split 2, 172 do not split.
+    // split (one for every wave group): 32 tiles on 256 CUs split 8, 86 split
+    // 2, 172 do not split.
     int splits = std::max(1, cus / tiles);
-    splits = std::min(splits, std::max(1, p.nb / 2));
+    splits = std::min(splits, std::max(1, p.nb / (KG > 1 ? KG : 2)));
     if (tuning().gemm_splits) splits = tuning().gemm_splits;
     // the fp32 partials (one TM x 256 tile per unit) must fit the scratch
     const size_t unit_bytes = (size_t)TM * RPW * sizeof(float);
@@ -1016,7 +1070,7 @@ static hipError_t launch_gemm_t(void *y, const uint8_t *w, const uint16_t *x, in
     const double x_bytes = 2.0 * N * K, w_bytes = (double)M * row_bytes;
     p.tok_major = tuning().gemm_order ? tuning().gemm_order == 2
                                       : x_bytes + p.tok_tiles * w_bytes < 8 * x_bytes + w_bytes;
-    gemm_kernel<T, XT, YT, TM, NW><<<8 * p.units_per_xcd, THREADS, 0, st>>>(p);
+    gemm_kernel<T, XT, YT, TM, NW, KG><<<8 * p.units_per_xcd, THREADS * KG, 0, st>>>(p);
     if (splits > 1) {  // 4 * TM / 32 float4 per thread; at most units_per_xcd / splits + 1 tiles per XCD
         constexpr int E = 4 * (TM / 32);
         gemm_reduce_kernel<YT, TM, NW>
@@ -1078,6 +1132,29 @@ static hipError_t launch_gemm_tm(void *y, const uint8_t *w, const uint16_t *x, i
                                  int K, hipStream_t st, const Scratch &sc) {
     int tm = tuning().gemm_tm;
     int big = -1;  // whole areas per XCD for the mixed kernel
+    // Up to 64 tokens: token tiles of 32 or 64 and two or four wave groups that
+    // share K, instead of 128-token tiles mostly of padding on few workgroups.
+    // 64-row tiles (two waves, four groups) where they fill a quarter of the
+    // CUs or more in one round, 128-row tiles (four waves, two groups)
+    // otherwise.  Measured against the 128-token tiles, Q4_K, 17 / 45 tokens,
+    // us: [256 x 2048] 11.7 -> 7.4 / 8.2, [2048 x 2048] 14.1 -> 8.6 / 9.9,
+    // [11008 x 2048] 23.1 -> 10.3 / 12.7 (12.6 / 15.6 with 128 rows), [4096 x
+    // 4096] 18.2 -> 10.2 / 12.8 (10.9 / 14.1), [2048 x 11008] 20.1 -> 13.0 /
+    // 16.3, [28672 x 4096] 43 -> 22.4 / 28.3 (25.6 / 36.1 with 64 rows);
+    // Q5_K alike, Q6_K 45 tokens [11008 x 2048] 25.5 -> 20.6, [28672 x 4096]
+    // 57.5 -> 47.4.  65 tokens in two tiles are no faster than one of 128.
+    // RXQ4_GEMM_* ask for the larger tiles.
+    const Tuning &t = tuning();
+    if (N <= 64 && !t.gemm_splits && !t.gemm_tm && !t.gemm_order && !t.gemm_mixed && !t.gemm_nw) {
+        const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
+        const int tiles64 = (M + 63) / 64;
+        if (tiles64 <= cus && 4 * tiles64 >= cus) {
+            if (N <= 32) return launch_gemm_t<T, XT, YT, 32, 2, 4>(y, w, x, M, N, K, st, sc);
+            return launch_gemm_t<T, XT, YT, 64, 2, 4>(y, w, x, M, N, K, st, sc);
+        }
+        if (N <= 32) return launch_gemm_t<T, XT, YT, 32, 4, 2>(y, w, x, M, N, K, st, sc);
+        return launch_gemm_t<T, XT, YT, 64, 4, 2>(y, w, x, M, N, K, st, sc);
+    }
     if (tm != 128 && tm != 256) {
         const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
         const int c = std::max(1, cus / 8);  // CUs per XCD
@@ -1221,10 +1298,7 @@ static hipError_t launch_tokens_t(void *y, const uint8_t *w, const uint16_t *x, 
         }
         gemv_tokens_lds_kernel<XT, YT, 1, 4>
             <<<dim3(g64, splits), 256, 0, st>>>(y, w, x, M, n_tok, K, ws, sbps);
-        if (splits > 1) {
-            const int64_t n = (int64_t)n_tok * M;
-            tokens_reduce_kernel<YT><<<(unsigned)((n + 255) / 256), 256, 0, st>>>(y, ws, n, splits);
-        }
+        if (splits > 1) return launch_tokens_reduce(y, YT, ws, (int64_t)n_tok * M, splits, st);
         return hipGetLastError();
     }
     // Short rows (nb < 16): the register kernel, never split over K (every

@@ -847,7 +847,8 @@ template <int T, int XT, int YT, int RT, int TT>
 __global__ __launch_bounds__(256) void kq_tokens_kernel(void *__restrict__ y,
                                                         const uint8_t *__restrict__ w,
                                                         const uint16_t *__restrict__ x, int M,
-                                                        int N, int K) {
+                                                        int N, int K, float *__restrict__ ws,
+                                                        int b_per_split) {
     constexpr int BYTES = KqFormat<T>::kBytes;
     constexpr int NF = RT * TT;  // 16 x 16 output fragments per wave
     __shared__ f32x4 part[4][NF][64];
@@ -869,7 +870,8 @@ __global__ __launch_bounds__(256) void kq_tokens_kernel(void *__restrict__ y,
         for (int t = 0; t < TT; ++t) acc[r][t] = f32x4{0.f, 0.f, 0.f, 0.f};
     // K blocks round-robin over the 4 waves; each block's RT weight
     // fragments are dequantised once and used for all TT token fragments.
-    for (int b = wave; b < nb; b += 4) {
+    const int b_end = min(nb, (int)(blockIdx.z + 1) * b_per_split);  // K split blockIdx.z
+    for (int b = blockIdx.z * b_per_split + wave; b < b_end; b += 4) {
         u32x4 a[RT][8];
 #pragma unroll
         for (int r = 0; r < RT; ++r)
@@ -905,54 +907,71 @@ __global__ __launch_bounds__(256) void kq_tokens_kernel(void *__restrict__ y,
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int row = 16 * r + 4 * g + q;
-                if (row < n_rows) store_out<YT>(y, (int64_t)(tok0 + tok) * M + row0 + row, s[q]);
+                if (row >= n_rows) continue;
+                const int64_t at = (int64_t)(tok0 + tok) * M + row0 + row;
+                if (ws) ws[(int64_t)blockIdx.z * N * M + at] = s[q];
+                else store_out<YT>(y, at, s[q]);
             }
         }
     }
 }
 
-template <int T, int XT, int YT, int RT, int TT>
-static void launch_kq_tok(dim3 grid, void *y, const uint8_t *w, const uint16_t *x, int M, int N,
-                          int K, hipStream_t st) {
-    kq_tokens_kernel<T, XT, YT, RT, TT><<<grid, 256, 0, st>>>(y, w, x, M, N, K);
-}
-
-// Small batches (the C ABI sends more than 16 tokens to the eight-wave GEMM
-// of gemm_q4k.hip): one 16-token fragment per workgroup (grid.y walks the
-// 16-token chunks), 32 rows when that still gives a workgroup per CU.
+// Small batches (the C ABI sends more than 16 tokens to the GEMM of
+// gemm_q4k.hip): one 16-token fragment per workgroup (grid.y walks the
+// 16-token chunks), 32 rows when that still gives a workgroup per CU.  With
+// fewer workgroups than four per CU, rows of 20 blocks or more are split over
+// workgroups, a wave keeping at least two blocks (one block after another per
+// wave, each a memory round trip and its dequantisation): [2048 x 11008] at 4 /
+// 16 tokens, Q6_K 24.1 / 27.3 -> 13.2 / 15.7 us, Q5_K 20.6 / 23.2 -> 11.0 /
+// 13.7, Q6_K [4096 x 14336] 29.2 / 33.6 -> 22.5 / 28.2, [5120 x 5120] 16.3 /
+// 19.9 -> 14.6 / 17.9; rows of 16 blocks 10.4 / 10.4 -> 10.0 / 11.5 (unsplit).
 template <int T, int XT, int YT>
 static hipError_t launch_kq_tokens_xy(void *y, const uint8_t *w, const uint16_t *x, int M, int N,
-                                      int K, hipStream_t st) {
+                                      int K, hipStream_t st, const Scratch &sc) {
     const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
-    const int chunks = (N + 15) / 16;
+    const int chunks = (N + 15) / 16, nb = K / 256;
     const int rt = (int64_t)((M + 31) / 32) * chunks >= cus ? 2 : 1;
-    const dim3 grid((M + 16 * rt - 1) / (16 * rt), chunks);
+    const int64_t wgs = (int64_t)((M + 16 * rt - 1) / (16 * rt)) * chunks;
+    int splits = nb < 20 ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(4 * (int64_t)cus / wgs, nb / 8));
+    if (tuning().tokens_lds_split) splits = std::min(tuning().tokens_lds_split, nb);
+    splits = (int)std::min<size_t>(splits, std::max<size_t>(1, sc.capacity() / ((size_t)N * M * sizeof(float))));
+    int per = (nb + splits - 1) / splits;
+    splits = (nb + per - 1) / per;
+    float *ws = nullptr;
+    if (splits > 1 && sc.get(st, (size_t)splits * N * M * sizeof(float), &ws) != hipSuccess) {
+        (void)hipGetLastError();  // no workspace: the unsplit plan needs none
+        ws = nullptr;
+        splits = 1;
+        per = nb;
+    }
+    const dim3 grid((M + 16 * rt - 1) / (16 * rt), chunks, splits);
     if (grid.y > 65535) return hipErrorInvalidValue;
-    if (rt == 2) launch_kq_tok<T, XT, YT, 2, 1>(grid, y, w, x, M, N, K, st);
-    else launch_kq_tok<T, XT, YT, 1, 1>(grid, y, w, x, M, N, K, st);
+    if (rt == 2) kq_tokens_kernel<T, XT, YT, 2, 1><<<grid, 256, 0, st>>>(y, w, x, M, N, K, ws, per);
+    else kq_tokens_kernel<T, XT, YT, 1, 1><<<grid, 256, 0, st>>>(y, w, x, M, N, K, ws, per);
+    if (splits > 1) return launch_tokens_reduce(y, YT, ws, (int64_t)N * M, splits, st);
     return hipGetLastError();
 }
 
 template <int T>
 static hipError_t launch_kq_tokens_t(void *y, int y_dtype, const uint8_t *w, const void *x,
-                                     int x_dtype, int M, int N, int K, hipStream_t st) {
+                                     int x_dtype, int M, int N, int K, hipStream_t st, const Scratch &sc) {
     const int64_t row_bytes = (int64_t)(K / 256) * KqFormat<T>::kBytes;
     if (row_bytes * 32 > 0x7FFFFFFF || (int64_t)128 * K * 2 > 0x7FFFFFFF) return hipErrorInvalidValue;
     const uint16_t *xx = static_cast<const uint16_t *>(x);
     if (x_dtype == RXQ4_DTYPE_BF16) {
         if (y_dtype == RXQ4_DTYPE_BF16)
-            return launch_kq_tokens_xy<T, RXQ4_DTYPE_BF16, RXQ4_DTYPE_BF16>(y, w, xx, M, N, K, st);
-        return launch_kq_tokens_xy<T, RXQ4_DTYPE_BF16, RXQ4_DTYPE_F32>(y, w, xx, M, N, K, st);
+            return launch_kq_tokens_xy<T, RXQ4_DTYPE_BF16, RXQ4_DTYPE_BF16>(y, w, xx, M, N, K, st, sc);
+        return launch_kq_tokens_xy<T, RXQ4_DTYPE_BF16, RXQ4_DTYPE_F32>(y, w, xx, M, N, K, st, sc);
     }
     if (y_dtype == RXQ4_DTYPE_F16)
-        return launch_kq_tokens_xy<T, RXQ4_DTYPE_F16, RXQ4_DTYPE_F16>(y, w, xx, M, N, K, st);
-    return launch_kq_tokens_xy<T, RXQ4_DTYPE_F16, RXQ4_DTYPE_F32>(y, w, xx, M, N, K, st);
+        return launch_kq_tokens_xy<T, RXQ4_DTYPE_F16, RXQ4_DTYPE_F16>(y, w, xx, M, N, K, st, sc);
+    return launch_kq_tokens_xy<T, RXQ4_DTYPE_F16, RXQ4_DTYPE_F32>(y, w, xx, M, N, K, st, sc);
 }
 
 hipError_t launch_kq_tokens(int ggml_type, void *y, int y_dtype, const uint8_t *w, const void *x,
-                            int x_dtype, int M, int N, int K, hipStream_t st) {
-    if (ggml_type == 14) return launch_kq_tokens_t<14>(y, y_dtype, w, x, x_dtype, M, N, K, st);
-    if (ggml_type == 13) return launch_kq_tokens_t<13>(y, y_dtype, w, x, x_dtype, M, N, K, st);
+                            int x_dtype, int M, int N, int K, hipStream_t st, const Scratch &sc) {
+    if (ggml_type == 14) return launch_kq_tokens_t<14>(y, y_dtype, w, x, x_dtype, M, N, K, st, sc);
+    if (ggml_type == 13) return launch_kq_tokens_t<13>(y, y_dtype, w, x, x_dtype, M, N, K, st, sc);
     return hipErrorInvalidValue;
 }
 

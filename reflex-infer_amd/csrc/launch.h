@@ -119,9 +119,14 @@ hipError_t launch_kq_gemv(int ggml_type, const GemvRange &r, const uint16_t *x, 
 hipError_t launch_kq_multi(const GemvRange *ranges, const int *types, int n_ranges,
                            const uint16_t *x, int K, hipStream_t stream);
 
-// Q5_K / Q6_K multi-token product for any N >= 1 (16-token chunks).
+// Q5_K / Q6_K multi-token product for any N >= 1 (16-token chunks; K split over
+// workgroups, through `sc`, where a few rows of many super-blocks leave CUs idle).
 hipError_t launch_kq_tokens(int ggml_type, void *y, int y_dtype, const uint8_t *w, const void *x,
-                            int x_dtype, int M, int N, int K, hipStream_t stream);
+                            int x_dtype, int M, int N, int K, hipStream_t stream,
+                            const Scratch &sc = Scratch{});
+// y[i] (y_dtype) = sum over the splits, in order, of ws[split][i], i < n.
+hipError_t launch_tokens_reduce(void *y, int y_dtype, const float *ws, int64_t n, int splits,
+                                hipStream_t stream);
 
 // Q6_K embedding rows (as launch_embed).
 hipError_t launch_kq_embed(uint16_t *dst, const uint8_t *w, const int32_t *ids, int token_id,

@@ -216,9 +216,14 @@ int gemm_impl(const char *fn, void *y, int y_dtype, const void *w, int ggml_type
                            y_dtype == RXQ4_DTYPE_F32 ? rxq4::kEpiF32 : rxq4::kEpiF16, stream);
     }
     hipError_t e;
-    if (kquant_type(ggml_type) && N <= rxq4::kMaxSmallBatch)
+    // Q5_K matrices of 200000 blocks or more go to the GEMM's 32-token tiles at
+    // any token count ([28672 x 4096] at 4 / 16 tokens 32.5 / 39.2 -> 25.2 / 25.7
+    // us, [4096 x 14336] 21.0 / 28.1 -> 18.2 / 18.7; [5120 x 5120] 12.7 / 16.5
+    // against 14.1 / 14.1; Q6_K [28672 x 4096] 40.1 / 44.6 against 43.6 / 43.5)
+    if (kquant_type(ggml_type) && N <= rxq4::kMaxSmallBatch &&
+        !(ggml_type == RXQ4_GGML_TYPE_Q5_K && (int64_t)M * (K / 256) >= 200000))
         e = rxq4::launch_kq_tokens(ggml_type, y, y_dtype, static_cast<const uint8_t *>(w), x,
-                                   x_dtype, M, N, K, st);
+                                   x_dtype, M, N, K, st, sc);
     else if (kquant_type(ggml_type))
         e = rxq4::launch_gemm(ggml_type, y, y_dtype, static_cast<const uint8_t *>(w), x, x_dtype,
                               M, N, K, st, sc);

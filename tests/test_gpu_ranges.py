@@ -10,6 +10,7 @@ import torch
 
 from oracle import oracle as orc
 from rxq4 import capi
+from tests import kquant_blocks as kb
 from tests import util
 
 pytestmark = pytest.mark.gpu
@@ -119,3 +120,64 @@ def test_prefill_attention_split_in_a_graph():
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
     capi.release_workspace(stream)
+
+
+# ------------------------------------------------------- 17..64 token products
+# Token tiles of 32 and 64 on 128-row tiles (two wave groups share K) and, from
+# 64 row tiles of 64 rows, on 64-row tiles (four groups): groups without
+# super-blocks (K of one to three), uneven parts, K splits, partial row tiles,
+# rows that no vector store covers, the first and last token count of a tile.
+SHORT = [(12, 1, 17, 256), (12, 130, 32, 256), (12, 129, 33, 512), (12, 300, 64, 768), (12, 257, 45, 2048),
+         (12, 64, 20, 11008), (12, 4100, 31, 1280), (12, 4101, 47, 256), (12, 4160, 64, 2816),
+         (13, 130, 17, 512), (13, 131, 50, 2304), (13, 4099, 64, 768), (13, 200, 60, 5120),
+         (14, 1, 64, 256), (14, 130, 32, 768), (14, 133, 33, 2304), (14, 4102, 17, 1280), (14, 60, 64, 11008)]
+
+
+def product_case(t, M, N, K, dt, seed):
+    Wn = util.weights(seed, M, K) if t == 12 else kb.random_blocks(t, util.rng(seed), M, K)
+    x32 = util.gaussian(seed + 1, (N, K))
+    if dt == "bf16":
+        bits = util.f32_to_bf16_bits(x32)
+        x, xf = dev(bits).view(torch.bfloat16), orc.bits_bf16_to_f32(bits)
+    else:
+        bits = x32.astype(np.float16).view(np.uint16)
+        x, xf = dev(bits).view(torch.float16), orc.bits_f16(bits).astype(np.float32)
+    rows = np.unique(np.r_[0, np.arange(max(0, M - 40), M), util.rng(seed + 2).choice(M, min(M, 60), replace=False)])
+    sub = np.ascontiguousarray(Wn[rows])
+    ref = orc.gemm_f64(sub, K, xf, dt) if t == 12 else orc.kq_gemm_f64(sub, K, t, xf, dt)
+    return dev(Wn), x, rows, ref
+
+
+def check_product(call, W, x, rows, ref, t, M, N, K, dt):
+    y = torch.full((N, M), float("nan"), dtype=torch.float32, device="cuda")
+    call(y, W, x, M, N, K, ggml_type=t)
+    assert util.rel_err(y.cpu().numpy()[:, rows], ref) <= util.TOL
+    assert torch.isfinite(y).all()
+    y16 = torch.empty((N, M), dtype=x.dtype, device="cuda")
+    call(y16, W, x, M, N, K, ggml_type=t)
+    assert util.rounded_ok(host16(y16)[:, rows], ref, dt).all()
+
+
+@pytest.mark.parametrize("t,M,N,K", SHORT)
+def test_short_prompt_products(t, M, N, K):
+    print(f"short prompt type {t} [{M} x {K}] x {N}", flush=True)
+    for dt in ("f16", "bf16"):
+        case = product_case(t, M, N, K, dt, 7300 + M + N)
+        check_product(capi.gemm, *case, t, M, N, K, dt)
+        check_product(capi.gemm_noalloc, *case, t, M, N, K, dt)
+
+
+# Q5_K / Q6_K batches whose rows are split over workgroups (20 blocks a row and
+# up; parts of 2 to 11 blocks, the last one short), the largest unsplit row,
+# and Q5_K batches large enough for the 32-token tiles.
+BATCH = [(14, 100, 2, 5120), (14, 33, 16, 11008), (13, 33, 5, 11008), (13, 16, 16, 5376), (14, 64, 7, 4864),
+         (14, 2049, 3, 5120), (13, 12501, 2, 4096), (13, 12500, 16, 4096)]
+
+
+@pytest.mark.parametrize("t,M,N,K", BATCH)
+def test_kquant_batches_split_and_large(t, M, N, K):
+    print(f"kquant batch type {t} [{M} x {K}] x {N}", flush=True)
+    for dt in ("f16", "bf16"):
+        case = product_case(t, M, N, K, dt, 7400 + M + N)
+        check_product(capi.gemm, *case, t, M, N, K, dt)
+        check_product(capi.gemm_noalloc, *case, t, M, N, K, dt)
