@@ -983,6 +983,160 @@ __global__ __launch_bounds__(64 * kLdsStreamWaves) void gemv_lds_stream_kernel(G
     }
 }
 
+// ---------------------------------------------------------------------------
+// Row-group kernel, for rows whose slot count fills 64 lanes badly (K = 5120:
+// 80 slots, 62%; K = 1536: 24 slots, 37%): LPR lanes (8, 16 or 32) take a row,
+// so a wave takes RPG = 64 / LPR consecutive rows at once and walks their slots
+// LPR at a time (80 slots: five full steps of 16).  x is staged once per
+// workgroup as in the LDS kernel (a lane's slot changes every step); the lanes
+// of a row are summed once per row with DPP.  Two batches of U items in flight
+// per wave, about four waves per CU.  Bound: the stream of weights beside the
+// lanes' dot products, which idle lanes stretched.  Measured against the
+// kernels below (graph replay): [27648 x 5120] 26.1 -> 18.3 us (4.4 TB/s),
+// [17920 x 1536] 10.1 -> 6.7, [37888 x 3584] 22.4 -> 17.5, [5120 x 5120] 8.8 ->
+// 6.6, [4096 x 14336] 11.6 -> 9.3, [16384 x 3072] 12.0 -> 8.2, [1536 x 1536]
+// 3.8 -> 3.2.
+template <int EPI, int U, int NT, int LPR>
+__global__ __launch_bounds__(256) void gemv_rows_kernel(GemvParams p) {
+    constexpr int RPG = 64 / LPR;
+    extern __shared__ uint32_t xlds[];
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int sub = lane / LPR, sl = lane % LPR;
+    const int n_slots = 4 * p.nb;
+    const int J = (n_slots + LPR - 1) / LPR;
+    const int wave = blockIdx.x * 4 + wv;
+    const bool active = wave < p.total_units;
+    const Range rg = range_of_unit(p, active ? wave : 0);
+    const int n_groups = (rg.rows + RPG - 1) / RPG;
+    const int g0 = active ? (wave - rg.first_unit) * p.per_unit : 0;
+    const int g1 = active ? min(g0 + p.per_unit, n_groups) : 0;
+    const int n_items = (g1 - g0) * J;
+    const uint32_t row_bytes = (uint32_t)p.nb * kBlockBytes;
+    const int last = rg.rows - 1;
+
+    // Items (group, step) in order, loads up to two batches ahead.  Rows past
+    // the range re-read its last row, steps past the wave's last group repeat
+    // that group: loads are unconditional and in the range, results discarded.
+    int ld_g = g0, ld_j = 0;
+    auto row_of = [&](int g) { return min(max(0, min(g, g1 - 1)) * RPG + sub, last); };
+    const uint8_t *ld_row = rg.w + (int64_t)row_of(g0) * row_bytes;
+    auto load = [&](Batch<U> &bt) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int slot = min(LPR * ld_j + sl, n_slots - 1);
+            const uint8_t *blk = ld_row + (slot >> 2) * kBlockBytes;
+            bt.h[u] = load16(blk);
+            bt.a[u] = load16(blk + 16 + 32 * (slot & 3));
+            bt.c[u] = load16(blk + 32 + 32 * (slot & 3));
+            if (++ld_j == J) {
+                ld_j = 0;
+                ++ld_g;
+                ld_row = rg.w + (int64_t)row_of(ld_g) * row_bytes;
+            }
+        }
+    };
+    const int K = 256 * p.nb;
+    auto stage = [&](int s, const u32x4 raw[8]) {
+        XSlot xs;
+        x_slot_from_raw(raw, xs);
+        uint32_t *dst = xlds + s * kLdsSlotWords;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            *reinterpret_cast<u32x4 *>(dst + 4 * k) =
+                u32x4{xs.p[4 * k], xs.p[4 * k + 1], xs.p[4 * k + 2], xs.p[4 * k + 3]};
+        *reinterpret_cast<f32x4v *>(dst + 32) = f32x4v{xs.bias_lo, xs.bias_hi, xs.sx_lo, xs.sx_hi};
+    };
+    const int s_first = threadIdx.x;
+    const int s_load = min(s_first, n_slots - 1);
+    u32x4 xraw[NT][8];
+#pragma unroll
+    for (int tk = 0; tk < NT; ++tk) load_x_raw(p.x + (int64_t)tk * K, s_load >> 2, s_load & 3, xraw[tk]);
+    __builtin_amdgcn_sched_barrier(0);
+    Batch<U> A, B;
+    load(A);
+    load(B);
+    __builtin_amdgcn_sched_barrier(0);
+    if (s_first < n_slots) {
+#pragma unroll
+        for (int tk = 0; tk < NT; ++tk) stage(tk * n_slots + s_first, xraw[tk]);
+    }
+    for (int s = s_first + blockDim.x; s < n_slots; s += blockDim.x) {
+#pragma unroll
+        for (int tk = 0; tk < NT; ++tk) {
+            load_x_raw(p.x + (int64_t)tk * K, s >> 2, s & 3, xraw[0]);
+            stage(tk * n_slots + s, xraw[0]);
+        }
+    }
+    wait_lgkmcnt0();
+    lds_barrier();
+    if (n_items == 0) return;
+
+    const uint32_t magic = magic_vgpr();
+    float acc[NT];
+#pragma unroll
+    for (int tk = 0; tk < NT; ++tk) acc[tk] = 0.0f;
+    int cp_item = 0, cp_g = g0, cp_j = 0;
+    auto compute = [&](const Batch<U> &bt) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (cp_item < n_items) {  // uniform
+                const int slot = LPR * cp_j + sl;
+                const bool valid = slot < n_slots;
+                const int sx = valid ? slot : 0;
+                XSlot xs[NT];
+#pragma unroll
+                for (int tk = 0; tk < NT; ++tk) {
+                    const uint32_t *src = xlds + (tk * n_slots + sx) * kLdsSlotWords;
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) {
+                        const u32x4 v = *reinterpret_cast<const u32x4 *>(src + 4 * k);
+                        xs[tk].p[4 * k] = v.x; xs[tk].p[4 * k + 1] = v.y;
+                        xs[tk].p[4 * k + 2] = v.z; xs[tk].p[4 * k + 3] = v.w;
+                    }
+                    const f32x4v t = *reinterpret_cast<const f32x4v *>(src + 32);
+                    xs[tk].bias_lo = t[0];
+                    xs[tk].bias_hi = t[1];
+                    xs[tk].sx_lo = t[2];
+                    xs[tk].sx_hi = t[3];
+                }
+                const ScaleDecode sd = scale_decode_for(sx & 3);
+                float v[NT];
+                if (NT == 1)
+                    v[0] = slot_dot(bt.h[u], bt.a[u], bt.c[u], xs[0], sd, magic);
+                else
+                    slot_dot_nt<NT>(bt.h[u], bt.a[u], bt.c[u], xs, sd, magic, v);
+#pragma unroll
+                for (int tk = 0; tk < NT; ++tk) acc[tk] += valid ? v[tk] : 0.0f;
+                ++cp_item;
+                if (++cp_j == J) {
+                    const int row = cp_g * RPG + sub;
+                    const bool mine = sl == LPR - 1 && row <= last;
+                    uint32_t res = 0;
+                    if (EPI == kEpiAdd) res = rg.res[min(row, last)];
+#pragma unroll
+                    for (int tk = 0; tk < NT; ++tk) {
+                        const float total = lane_group_sum<LPR>(acc[tk]);
+                        if (mine) store_row<EPI>(rg, row, total, res, (int64_t)tk * p.y_stride);
+                        acc[tk] = 0.0f;
+                    }
+                    cp_j = 0;
+                    ++cp_g;
+                }
+            }
+        }
+    };
+    int i = 0;
+    for (; i + 2 * U < n_items; i += 2 * U) {
+        compute(A);
+        load(A);
+        compute(B);
+        load(B);
+    }
+    compute(A);
+    compute(B);
+}
+
 const DeviceInfo &device_info() {
     static thread_local int cached_dev = -1;
     static thread_local DeviceInfo info{0, 0};
@@ -1106,6 +1260,51 @@ static hipError_t launch_reg(const GemvParams &p, int grid, hipStream_t st) {
     return hipSuccess;
 }
 
+// Lanes per row of the row-group kernel, or 64 for the kernels that give a row
+// the whole wave: the fewest 64-lane items that the busiest of 4 waves per CU
+// has, per wave the groups of 64 / LPR rows it takes times a group's steps.
+// Ties go to more rows a wave (fewer sums: [8192 x 8192], 16 items either way,
+// 9.7 us with 8 lanes, 10.6 with 64), but to the whole wave where it takes at
+// most two rows (the streamed kernel's one-row waves, two a SIMD: down [2048 x
+// 11008] 5.5-5.9 against 5.7 us with 32 lanes).  Other items against times, 8 /
+// 16 / 32 lanes: [5120 x 13824] 27 / 28 / 21 (64 lanes: 20), 13.2 / 13.6 / 11.6
+// (11.4) us; [4096 x 14336] 28 / 14 / 14, 13.0 / 9.3 / 9.7; [1536 x 8960] 18 /
+// 9 / 5, 8.5 / 6.0 / 4.8.  Rows and length alone decide, so every token count
+// sums a row in the same order.
+static int row_lanes(int64_t rows, int nb, int cus) {
+    const int64_t waves = 4 * (int64_t)cus;
+    int best = 64;
+    int64_t best_items = (rows + waves - 1) / waves * ((4 * nb + 63) / 64);
+    const bool whole = rows <= 2 * waves;
+    for (const int lpr : {32, 16, 8}) {
+        const int64_t groups = (rows + 64 / lpr - 1) / (64 / lpr);
+        const int64_t items = (groups + waves - 1) / waves * ((4 * nb + lpr - 1) / lpr);
+        if (items < best_items || (items == best_items && !(whole && best == 64))) {
+            best = lpr;
+            best_items = items;
+        }
+    }
+    return best;
+}
+
+template <int EPI, int NT, int LPR>
+static hipError_t launch_rows(const GemvParams &p, int grid, size_t lds, hipStream_t st) {
+    // the dynamic LDS limit (160 KB), raised once per device (devices 0..63)
+    static std::atomic<uint64_t> raised{0};
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    const uint64_t bit = 1ull << (dev & 63);
+    if (!(raised.load(std::memory_order_acquire) & bit)) {
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemv_rows_kernel<EPI, kRegBatch, NT, LPR>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        if (e != hipSuccess) return e;
+        raised.fetch_or(bit, std::memory_order_acq_rel);
+    }
+    gemv_rows_kernel<EPI, kRegBatch, NT, LPR><<<grid, 256, lds, st>>>(p);
+    return hipGetLastError();
+}
+
 template <int EPI, int NT>
 static hipError_t launch_gemv_epi(GemvParams p, hipStream_t st) {
     const int slots = 4 * p.nb;
@@ -1128,6 +1327,17 @@ static hipError_t launch_gemv_epi(GemvParams p, hipStream_t st) {
             default: e = launch_reg<64, EPI, NT>(p, grid, st); break;
         }
         if (e != hipSuccess) return e;
+    } else if (const int lpr = row_lanes(p.total_rows, p.nb, cus); lpr < 64) {
+        const size_t lds = (size_t)NT * slots * kLdsSlotWords * sizeof(uint32_t);
+        if (lds > 160 * 1024) return hipErrorInvalidValue;
+        const int rpg = 64 / lpr;
+        const int64_t target = (int64_t)cus * (tuning().gemv_lds_waves_per_cu ? tuning().gemv_lds_waves_per_cu : 4);
+        const int64_t groups = (p.total_rows + rpg - 1) / rpg;
+        const int waves = assign_units(p, rpg, (int)std::max<int64_t>(1, (groups + target - 1) / target));
+        const int grid = (waves + 3) / 4;
+        if (lpr == 8) return launch_rows<EPI, NT, 8>(p, grid, lds, st);
+        if (lpr == 16) return launch_rows<EPI, NT, 16>(p, grid, lds, st);
+        return launch_rows<EPI, NT, 32>(p, grid, lds, st);
     } else {
         // LDS kernels: whole rows per wave, `waves_per_cu` waves per CU (8
         // for the streamed kernel, 4 for the register-load kernel: down

@@ -181,3 +181,49 @@ def test_kquant_batches_split_and_large(t, M, N, K):
         case = product_case(t, M, N, K, dt, 7400 + M + N)
         check_product(capi.gemm, *case, t, M, N, K, dt)
         check_product(capi.gemm_noalloc, *case, t, M, N, K, dt)
+
+
+# --------------------------------------------------- decode GEMV, row groups
+# 8, 16 and 32 lanes a row: partial last groups of rows, steps past a row's
+# slots (a multiple of 4 only), several groups a wave, ranges of a pair and a
+# triple ending inside a group, 1 to 4 tokens, the residual in place.
+ROWS = [((5120,), 5120), ((27649,), 1280), ((17919,), 1536), ((1537,), 1536), ((1536,), 8960), ((4099,), 3584),
+        ((2047,), 3072), ((13823, 13825), 768), ((5121, 1, 1023), 5120), ((7, 9, 3), 2816), ((1,), 1792),
+        ((37890,), 3584), ((4097,), 14336), ((3,), 65280)]
+
+
+@pytest.mark.parametrize("rows,K", ROWS)
+def test_row_group_gemv(rows, K):
+    print(f"row groups {rows} x {K}", flush=True)
+    x = util.x_f16(7500, K)
+    xd, xf = dev(x).view(torch.float16), orc.bits_f16(x).astype(np.float32)
+    Ws = [util.weights(7501 + i, M, K) for i, M in enumerate(rows)]
+    Wd = [dev(W) for W in Ws]
+    ys = [torch.full((M,), float("nan"), dtype=torch.float16, device="cuda") for M in rows]
+    capi.gemv_multi_f16([(y, W, M) for y, W, M in zip(ys, Wd, rows)], xd, K)
+    picks = [np.unique(np.r_[0, M // 3, M // 2, np.arange(max(0, M - 70), M)]) for M in rows]
+    refs = [orc.gemv_f64(np.ascontiguousarray(W[p]), K, xf) for W, p in zip(Ws, picks)]
+    for y, p, ref in zip(ys, picks, refs):
+        assert torch.isfinite(y).all()
+        assert util.rounded_ok(host16(y)[p], ref).all()
+    M, W, p, ref = rows[0], Wd[0], picks[0], refs[0]
+    f32 = torch.empty(M, dtype=torch.float32, device="cuda")
+    capi.gemv_f32(f32, W, xd, M, K)
+    assert util.rel_err(f32.cpu().numpy()[p], ref) <= util.TOL
+    res = util.x_f16(7510, M)
+    rd = dev(res).view(torch.float16)
+    one = torch.empty(M, dtype=torch.float16, device="cuda")
+    capi.gemv_f16(one, W, xd, M, K)
+    expect = (one.float() + rd.float()).half()  # the product rounded, then the sum
+    capi.gemv_add_f16(rd, W, xd, rd, M, K)
+    assert torch.equal(rd, expect)
+    if K <= 8960:  # every token of a multi-token call equals its own call
+        xs = dev(util.x_f16(7520, (3, K))).view(torch.float16)
+        for N in (2, 3):
+            if not util.gemv_path(N, M, K):
+                continue
+            many = torch.empty((N, M), dtype=torch.float16, device="cuda")
+            capi.gemm_f16(many, W, xs, M, N, K)
+            for t in range(N):
+                capi.gemv_f16(one, W, xs[t], M, K)
+                assert torch.equal(many[t], one), (N, t)
