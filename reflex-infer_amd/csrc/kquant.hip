@@ -119,6 +119,15 @@ __device__ __forceinline__ float kq_row_sum(float v, int slots) {
     return v;
 }
 
+// The same for groups of 8, 16 or 32 lanes of the row groups, on the VALU.
+__device__ __forceinline__ float kq_lanes_sum(float v, int lanes) {
+    if (lanes == 32) return butterfly_sum<32>(v);
+    v = dpp_row_add<0xB1>(v);   // quad_perm [1,0,3,2]
+    v = dpp_row_add<0x4E>(v);   // quad_perm [2,3,0,1]
+    v = dpp_row_add<0x141>(v);  // row_half_mirror: the other quad of 8
+    return lanes == 16 ? dpp_row_add<0x128>(v) : v;  // row_ror:8
+}
+
 struct XLds {
     const u32x4 *x;   // 8 fp16 per element
     const float *sum;
@@ -268,8 +277,9 @@ struct KqGemvParams {
     const uint16_t *x;
     int M, K, nb, row_bytes;
     int slots;     // 4 * nb
-    int rows_per;  // rows per wave step (64 / slots) or 0: one row per step
-    int n_units;   // wave steps (packed rows) or rows
+    int rows_per;  // rows per wave step (64 / slots) or 0
+    int lanes;     // row groups: lanes per row (32, 16 or 8), else 0
+    int n_units;   // wave steps (packed rows), rows or row groups
 };
 
 template <int T>
@@ -317,10 +327,11 @@ __device__ __forceinline__ uint32_t kq_res(const KqGemvParams &p, int row) {
     return EPI == kEpiAdd ? p.res[min(row, p.M - 1)] : 0u;
 }
 
-// PACKED: rows of at most 64 slots packed into wave steps (p.rows_per > 0);
-// else one row per wave.  Two instances, so that each path gets its own
-// register allocation.
-template <int T, int EPI, bool PACKED>
+// Packed: rows of at most 64 slots packed into wave steps (p.rows_per > 0);
+// whole: one row per wave; groups: 64 / p.lanes rows per wave.  Instances, so
+// that each path gets its own register allocation.
+enum KqRows { kKqWhole, kKqPacked, kKqGroups };
+template <int T, int EPI, KqRows ROWS>
 __global__ __launch_bounds__(256) void kq_gemv_kernel(KqGemvParams p) {
     constexpr int BYTES = KqFormat<T>::kBytes;
     extern __shared__ u32x4 kq_smem[];
@@ -349,7 +360,7 @@ __global__ __launch_bounds__(256) void kq_gemv_kernel(KqGemvParams p) {
         }
         __syncthreads();
     };
-    if constexpr (PACKED) {
+    if constexpr (ROWS == kKqPacked) {
         // slots = 64 / rows_per lanes per row; the wave takes the steps
         // wave_g + k * n_waves.  Two steps are in flight at all times: step
         // k + 2 is issued as soon as step k has been computed.  Steps past
@@ -390,6 +401,72 @@ __global__ __launch_bounds__(256) void kq_gemv_kernel(KqGemvParams p) {
                 load(st + 2 * n_waves, A);
                 finish(B);
                 load(st + 3 * n_waves, B);
+            }
+            finish(A);
+            finish(B);
+        }
+    } else if constexpr (ROWS == kKqGroups) {
+        // Row groups: p.lanes lanes a row, so 64 / lanes rows at once, their
+        // slots `lanes` at a time (a whole wave leaves 48 lanes idle
+        // in every other step of an 80-slot row).  The wave's groups wave_g + k *
+        // n_waves and their steps are one stream of items with two in flight;
+        // items past it repeat its last group, slots past a row its last
+        // block: unconditional loads, results discarded.
+        const int lanes = p.lanes, rpg = 64 / lanes;
+        const int sub = lane / lanes, sl = lane - sub * lanes;
+        const int n_steps = (p.slots + lanes - 1) / lanes;
+        struct Item {
+            Slot<T> s;
+            int ex, j, unit;
+            uint32_t res;
+        };
+        int lu = wave_g, lj = 0;
+        auto place = [&](int j, int &u) {  // byte offset of the lane's slot in its row group
+            const int slot = j * lanes + sl;
+            u = slot & 3;
+            return sub * p.row_bytes + min(slot >> 2, p.nb - 1) * BYTES;
+        };
+        auto load = [&](Item &o) {
+            o.unit = lu;
+            o.j = lj;
+            const int r0 = min(lu, p.n_units - 1) * rpg;
+            const RowRes rr = row_rsrc(p.w + (int64_t)r0 * p.row_bytes, min(rpg, p.M - r0) * p.row_bytes);
+            o.ex = rr.ex;
+            int u;
+            const int off = place(lj, u);
+            o.s.load(rr.rs, rr.ex + off, u);
+            o.res = kq_res<EPI>(p, r0 + sub);
+            if (++lj == n_steps) {
+                lj = 0;
+                lu += n_waves;
+            }
+        };
+        float acc = 0.0f;
+        auto finish = [&](const Item &o) {
+            if (o.unit >= p.n_units) return;  // uniform
+            int u;
+            const int off = place(o.j, u), slot = o.j * lanes + sl;
+            const float v = o.s.dot(o.ex + off, u, min(slot >> 2, p.nb - 1) * 256, xl);
+            acc += slot < p.slots ? v : 0.0f;
+            if (o.j == n_steps - 1) {  // uniform
+                const float sum = kq_lanes_sum(acc, lanes);
+                const int row = o.unit * rpg + sub;
+                if (sl == 0 && row < p.M) kq_store<EPI>(p, row, sum, o.res);
+                acc = 0.0f;
+            }
+        };
+        stage_x();
+        if (wave_g < p.n_units) {
+            Item A, B;
+            load(A);
+            load(B);
+            const int n_items = (p.n_units - 1 - wave_g) / n_waves * n_steps + n_steps;
+            int i = 0;
+            for (; i + 2 < n_items; i += 2) {
+                finish(A);
+                load(A);
+                finish(B);
+                load(B);
             }
             finish(A);
             finish(B);
@@ -578,7 +655,7 @@ __global__ __launch_bounds__(256) void kq_multi_kernel(KqMultiParams p) {
     kq_multi_units(p, u0, lane, xl);
 }
 
-template <int T, int EPI, bool PACKED>
+template <int T, int EPI, KqRows ROWS>
 static hipError_t launch_kq_gemv_p(const KqGemvParams &p, hipStream_t st) {
     const size_t lds = (size_t)p.K * 2 + (size_t)(p.K / 16) * 4;
     if (lds > 160 * 1024) return hipErrorInvalidValue;
@@ -592,19 +669,39 @@ static hipError_t launch_kq_gemv_p(const KqGemvParams &p, hipStream_t st) {
     const int want = (p.n_units + 3) / 4;
     const int grid = std::max(1, std::min(want, cus * wg_per_cu));
     if (lds > 64 * 1024) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&kq_gemv_kernel<T, EPI, PACKED>),
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&kq_gemv_kernel<T, EPI, ROWS>),
                                                  hipFuncAttributeMaxDynamicSharedMemorySize,
                                                  (int)lds);
         if (e != hipSuccess) return e;
     }
-    kq_gemv_kernel<T, EPI, PACKED><<<grid, 256, lds, st>>>(p);
+    kq_gemv_kernel<T, EPI, ROWS><<<grid, 256, lds, st>>>(p);
     return hipGetLastError();
 }
 
 template <int T, int EPI>
 static hipError_t launch_kq_gemv_t(const KqGemvParams &p, hipStream_t st) {
-    return p.rows_per > 0 ? launch_kq_gemv_p<T, EPI, true>(p, st)
-                          : launch_kq_gemv_p<T, EPI, false>(p, st);
+    if (p.rows_per > 0) return launch_kq_gemv_p<T, EPI, kKqPacked>(p, st);
+    return p.lanes ? launch_kq_gemv_p<T, EPI, kKqGroups>(p, st) : launch_kq_gemv_p<T, EPI, kKqWhole>(p, st);
+}
+
+// Lanes per row for row groups, or 0 for a wave per row: with at least 40 rows
+// per CU (fewer leave too little work per wave: Q6_K [5120 x 5120] 8.8 us, in
+// groups 10.3-11.3; [6400 x 2560] 6.3 against 7.6), when a whole wave would idle
+// more than a third of its lanes (Q6_K) or a tenth (Q5_K, whose slot is
+// cheaper), the largest of 32, 16 and 8 that idles the fewest.  Measured, us:
+// [27648 x 5120] (80 slots) Q6_K 34.8 -> 28.7, Q5_K 28.9 -> 23.7; [17920 x 1536]
+// (24) 11.7 -> 9.8, 11.9 -> 8.0; [37888 x 3584] (56) Q5_K 25.5 -> 21.4, Q6_K
+// 25.6 against 28.4; [16384 x 3072] (48) Q5_K 12.6 -> 10.5, Q6_K 12.1 against
+// 12.9; full waves ([57344 x 8192], 128) Q6_K 73.1 against 75.8.
+static int kq_lanes(int ggml_type, int64_t rows, int slots) {
+    const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
+    auto steps64 = [&](int lanes) { return (slots + lanes - 1) / lanes * lanes; };  // lanes used or idle
+    if (rows < 40 * (int64_t)cus || slots * (ggml_type == 14 ? 3 : 10) > steps64(64) * (ggml_type == 14 ? 2 : 9))
+        return 0;
+    int best = 32;
+    for (const int lanes : {16, 8})
+        if (steps64(lanes) < steps64(best)) best = lanes;
+    return best;
 }
 
 hipError_t launch_kq_gemv(int ggml_type, const GemvRange &r, const uint16_t *x, int K,
@@ -620,9 +717,11 @@ hipError_t launch_kq_gemv(int ggml_type, const GemvRange &r, const uint16_t *x, 
     p.row_bytes = p.nb * (ggml_type == 14 ? KqFormat<14>::kBytes : KqFormat<13>::kBytes);
     p.slots = 4 * p.nb;
     p.rows_per = (p.slots <= 64 && 64 % p.slots == 0) ? 64 / p.slots : 0;
-    p.n_units = p.rows_per ? (p.M + p.rows_per - 1) / p.rows_per : p.M;
+    p.lanes = p.rows_per ? 0 : kq_lanes(ggml_type, p.M, p.slots);
+    const int per = p.rows_per ? p.rows_per : p.lanes ? 64 / p.lanes : 1;
+    p.n_units = (p.M + per - 1) / per;
     if (p.M <= 0) return hipSuccess;
-    if ((int64_t)p.rows_per * p.row_bytes > 0x7FFFFFFF) return hipErrorInvalidValue;
+    if ((int64_t)per * p.row_bytes > 0x7FFFFFFF) return hipErrorInvalidValue;
 #define RXQ4_KQ_EPI(T)                                                   \
     switch (epilogue) {                                                  \
         case kEpiF16: return launch_kq_gemv_t<T, kEpiF16>(p, st);        \

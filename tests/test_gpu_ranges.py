@@ -227,3 +227,27 @@ def test_row_group_gemv(rows, K):
             for t in range(N):
                 capi.gemv_f16(one, W, xs[t], M, K)
                 assert torch.equal(many[t], one), (N, t)
+
+
+# Q5_K / Q6_K row groups (10240 rows and more; 32, 16 and 8 lanes a row): odd
+# row counts, the first row count of the rule, rows on odd 2-byte boundaries.
+@pytest.mark.parametrize("t,M,K", [(13, 10240, 2560), (13, 10243, 1536), (14, 10241, 1280), (14, 12345, 1536),
+                                   (13, 20001, 3584), (14, 10247, 5120), (13, 11111, 3072), (14, 10241, 256 * 9)])
+def test_kquant_row_groups(t, M, K):
+    print(f"kquant row groups type {t} [{M} x {K}]", flush=True)
+    Wn = kb.random_blocks(t, util.rng(7600 + K), M, K)
+    x = util.x_f16(7601, K)
+    W, xd = dev(Wn), dev(x).view(torch.float16)
+    pick = np.unique(np.r_[0:9, M // 2, np.arange(M - 40, M), util.rng(7602).choice(M, 60, replace=False)])
+    ref = orc.kq_gemm_f64(np.ascontiguousarray(Wn[pick]), K, t, orc.bits_f16(x).astype(np.float32)[None], None)[0]
+    y = torch.full((M,), float("nan"), dtype=torch.float32, device="cuda")
+    capi.gemv_f32(y, W, xd, M, K, ggml_type=t)
+    assert torch.isfinite(y).all()
+    assert util.rel_err(y.cpu().numpy()[pick], ref) <= util.TOL
+    one = torch.empty(M, dtype=torch.float16, device="cuda")
+    capi.gemv_f16(one, W, xd, M, K, ggml_type=t)
+    assert util.rounded_ok(host16(one)[pick], ref).all()
+    res = dev(util.x_f16(7603, M)).view(torch.float16)
+    expect = (one.float() + res.float()).half()
+    capi.gemv_add_f16(res, W, xd, res, M, K, ggml_type=t)
+    assert torch.equal(res, expect)
