@@ -82,8 +82,17 @@ def _check(status: int, what: str) -> int:
     return status
 
 
+# torch's current stream as a raw handle, without the Stream object that
+# torch.cuda.current_stream() builds on every call (7.2 -> 4.1 us for a
+# gemv_f32 call; the smallest kernels take 2.6 us)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def _stream(stream) -> int:
     if stream is None:
+        if _raw_stream is not None and _device is not None and torch.cuda.is_initialized():
+            return _raw_stream(_device())
         return torch.cuda.current_stream().cuda_stream
     if isinstance(stream, torch.cuda.Stream):
         return stream.cuda_stream
