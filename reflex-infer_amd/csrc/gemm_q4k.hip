@@ -1254,14 +1254,22 @@ static hipError_t launch_tokens_t(void *y, const uint8_t *w, const uint16_t *x, 
     const int t2 = (M + 31) / 32;
     const bool wide = n_tok <= 8;
     const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
-    if ((M + 63) / 64 >= cus) {
+    // x staged in LDS from one 64-row workgroup per CU, for short rows (whose
+    // K the other kernel would deal to four waves, each reading its own x
+    // fragments) from half of that, and a third with more than 8 tokens: [11008
+    // x 2048] at 4 / 8 / 16 tokens 8.2 / 9.6 / 11.9 -> 7.9 / 7.9 / 8.4 us, [9728
+    // x 2560] 10.2 / 11.7 / 14.0 -> 8.7 / 8.7 / 9.2, [8960 x 1536] 6.9 / 7.4 / 9.0
+    // -> 6.2 / 6.1 / 6.4, [5632 x 2048] at 16 8.7 -> 7.6; below, [8192 x 2048]
+    // at 8 6.1 against 7.4, [4096 x 2048] at 16 6.0 against 7.6.
+    const int g64 = (M + 63) / 64;
+    const bool short_rows = nb < 16 && (g64 > cus / 2 || (n_tok > 8 && g64 >= 5 * cus / 16));
+    if (g64 >= cus || short_rows) {
         // Workgroups of W = 4, 6 or 8 waves (16 rows each), one per CU when
         // they fit: W minimises the rows of the busiest CU, 16 W times the
         // rounds of workgroups (ties to the larger W).  [22016 x 2048]: 230
         // workgroups of 96 rows (4 waves: 344 put two on 88 CUs; 8 waves:
         // 172 leave 84 CUs idle); m = 16: 13.5 / 11.8 / 11.1 us with 4 / 8 /
         // 6 waves.
-        const int g64 = (M + 63) / 64;
         int nw = tuning().tokens_waves;
         if (nw != 4 && nw != 6 && nw != 8) {
             int best = 0;
@@ -1284,7 +1292,6 @@ static hipError_t launch_tokens_t(void *y, const uint8_t *w, const uint16_t *x, 
     if (nb >= 16) {
         // Long rows: 64-row workgroups with x staged in LDS and K split over
         // workgroups (about one per CU, at least 4 super-blocks a split).
-        const int g64 = (M + 63) / 64;
         int splits = tuning().tokens_lds_split ? std::min(tuning().tokens_lds_split, nb)
                                                : std::max(1, std::min(cus / g64, nb / 4));
         splits = (int)std::min<size_t>(
@@ -1303,14 +1310,9 @@ static hipError_t launch_tokens_t(void *y, const uint8_t *w, const uint16_t *x, 
     }
     // Short rows (nb < 16): the register kernel, never split over K (every
     // row is at most 15 super-blocks, dealt to the waves of one workgroup).
-    if (t2 * kWaves >= 1024) {
-        const dim3 grid(t2, 1);
-        if (wide)
-            gemv_tokens_kernel<XT, YT, 2, kWaves, true>
-                <<<grid, kWaves * 64, 0, st>>>(y, w, x, M, n_tok, K, nullptr, nb);
-        else
-            gemv_tokens_kernel<XT, YT, 2, kWaves, false>
-                <<<grid, kWaves * 64, 0, st>>>(y, w, x, M, n_tok, K, nullptr, nb);
+    if (t2 * kWaves >= 1024 && wide) {  // (more tokens on as many rows: staged above)
+        gemv_tokens_kernel<XT, YT, 2, kWaves, true>
+            <<<dim3(t2, 1), kWaves * 64, 0, st>>>(y, w, x, M, n_tok, K, nullptr, nb);
     } else {
         const int t1 = (M + 15) / 16;
         if (wide)

@@ -167,6 +167,21 @@ def test_short_prompt_products(t, M, N, K):
         check_product(capi.gemm_noalloc, *case, t, M, N, K, dt)
 
 
+# Q4_K batches around the row counts from which x is staged in LDS.
+STAGED = [(12, 8192, 5, 768), (12, 8193, 4, 768), (12, 8193, 8, 2048), (12, 5056, 16, 512), (12, 5057, 9, 512),
+          (12, 5060, 16, 3840), (12, 9000, 3, 256)]
+
+
+@pytest.mark.parametrize("t,M,N,K", STAGED)
+def test_q4k_batches_staged(t, M, N, K):
+    print(f"batch [{M} x {K}] x {N}", flush=True)
+    for dt in ("f16", "bf16"):
+        case = product_case(t, M, N, K, dt, 7350 + M + N)
+        if dt == "f16" and util.gemv_path(N, M, K):
+            continue
+        check_product(capi.gemm, *case, t, M, N, K, dt)
+
+
 # Q5_K / Q6_K batches whose rows are split over workgroups (20 blocks a row and
 # up; parts of 2 to 11 blocks, the last one short), the largest unsplit row,
 # and Q5_K batches large enough for the 32-token tiles.
