@@ -738,7 +738,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_reduce_kernel(GemmParams p) {
 template <int XT, int YT, int RT, int KW, bool WIDE>
 __global__ __launch_bounds__(KW * 64) void gemv_tokens_kernel(
     void *__restrict__ y, const uint8_t *__restrict__ w, const uint16_t *__restrict__ x, int M,
-    int N, int K, float *__restrict__ ws, int sb_per_split) {
+    int n_tok, int K) {
     __shared__ f32x4 part[KW][RT][64];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -751,14 +751,12 @@ __global__ __launch_bounds__(KW * 64) void gemv_tokens_kernel(
     const uint8_t *wr[RT];
 #pragma unroll
     for (int t = 0; t < RT; ++t) wr[t] = w + min(row0 + 16 * t + li, M - 1) * row_bytes;
-    const __amdgpu_buffer_rsrc_t xr = make_rsrc(x, N * K * 2);
+    const int tok0 = blockIdx.y * 16, N = min(16, n_tok - tok0);  // this workgroup's tokens
+    const __amdgpu_buffer_rsrc_t xr = make_rsrc(x + (int64_t)tok0 * K, N * K * 2);
     // bytes; >= N*K*2 for tokens >= N
     const int xoff = li * K * 2 + (WIDE ? 128 * g : 16 * g);
-    // Super-blocks [sb_lo, sb_hi) of K split blockIdx.y (all of K without a
-    // split), dealt to the waves round-robin.
-    const int sb_lo = blockIdx.y * sb_per_split, sb_hi = min(nb, sb_lo + sb_per_split);
-    const int n_sb = sb_hi - sb_lo;
-    const int n_w = wave < n_sb ? (n_sb - 1 - wave) / KW + 1 : 0;  // super-blocks of this wave
+    // super-blocks of this wave, dealt round-robin
+    const int n_w = wave < nb ? (nb - 1 - wave) / KW + 1 : 0;
 
     // x element of k-step s (0..7) for this lane's group g, relative to the
     // super-block: WIDE 64g + 32*(s/4) + 8*(s%4); otherwise 64*(s/2) +
@@ -771,7 +769,7 @@ __global__ __launch_bounds__(KW * 64) void gemv_tokens_kernel(
         u32x4 b[8];
     };
     auto load = [&](int i, Sb &o) {
-        const int sb = min(sb_lo + wave + i * KW, sb_hi - 1);
+        const int sb = min(wave + i * KW, nb - 1);
 #pragma unroll
         for (int t = 0; t < RT; ++t) {
             const uint8_t *blk = wr[t] + sb * kBlockBytes;
@@ -845,11 +843,7 @@ __global__ __launch_bounds__(KW * 64) void gemv_tokens_kernel(
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int row = row0 + 16 * t + 4 * g + r;
-                if (row >= M) continue;
-                if (ws)  // split K: fp32 partial [split][token][row]
-                    ws[((int64_t)blockIdx.y * N + li) * M + row] = sum[r];
-                else
-                    store_out<YT>(y, (int64_t)li * M + row, sum[r]);
+                if (row < M) store_out<YT>(y, (int64_t)(tok0 + li) * M + row, sum[r]);
             }
         }
     }
@@ -1016,6 +1010,18 @@ __global__ __launch_bounds__(256) void tokens_reduce_kernel(void *__restrict__ y
     store_out<YT>(y, i, s);
 }
 
+// One row tile per workgroup and grid.y 16-token chunks.
+template <int XT, int YT>
+static hipError_t launch_tokens_chunks(void *y, const uint8_t *w, const uint16_t *x, int M, int n_tok,
+                                       int K, hipStream_t st) {
+    const dim3 grid((M + 15) / 16, (n_tok + 15) / 16);
+    if (n_tok <= 8)
+        gemv_tokens_kernel<XT, YT, 1, 4, true><<<grid, 256, 0, st>>>(y, w, x, M, n_tok, K);
+    else
+        gemv_tokens_kernel<XT, YT, 1, 4, false><<<grid, 256, 0, st>>>(y, w, x, M, n_tok, K);
+    return hipGetLastError();
+}
+
 hipError_t launch_tokens_reduce(void *y, int y_dtype, const float *ws, int64_t n, int splits,
                                 hipStream_t st) {
     const unsigned g = (unsigned)((n + 255) / 256);
@@ -1145,7 +1151,26 @@ static hipError_t launch_gemm_tm(void *y, const uint8_t *w, const uint16_t *x, i
     // 57.5 -> 47.4.  65 tokens in two tiles are no faster than one of 128.
     // RXQ4_GEMM_* ask for the larger tiles.
     const Tuning &t = tuning();
-    if (N <= 64 && !t.gemm_splits && !t.gemm_tm && !t.gemm_order && !t.gemm_mixed && !t.gemm_nw) {
+    const bool forced = t.gemm_splits || t.gemm_tm || t.gemm_order || t.gemm_mixed || t.gemm_nw;
+    // Small matrices (a layer's k and v): the small-batch kernels over 16-token
+    // chunks, one launch without K splits or partials, while the 16-row
+    // workgroups of all chunks stay within two and a quarter per CU (rows of 9
+    // to 16 super-blocks, whose waves walk three or four of them: one per CU).
+    // Against the tiles, 17 / 48 / 64 tokens, Q4_K: [256 x 2048] 7.3 / 8.2 / 8.3
+    // -> 5.4 / 5.5 / 5.5 us, [2048 x 2048] 8.7 / 9.8 / 9.9 -> 5.7 / 8.6 / 8.7,
+    // [1024 x 4096] 8.6 / 9.9 / 10.1 -> 8.4 / 8.6 / 8.6; Q6_K [256 x 2048] 9.4 /
+    // 10.4 / 10.3 -> 5.5; past the rule [6144 x 2048] 9.5 / 11.8 against 10.3 /
+    // 17.4, [3072 x 3072] at 48 11.5 against 16.6.
+    {
+        const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
+        const int64_t wgs = (int64_t)((M + 15) / 16) * ((N + 15) / 16);
+        const int nb = K / 256;
+        if (!forced && ((nb <= 8 && 4 * wgs <= 9 * cus) || (nb <= 16 && wgs <= cus))) {
+            if constexpr (T == 12) return launch_tokens_chunks<XT, YT>(y, w, x, M, N, K, st);
+            else return launch_kq_tokens(T, y, YT, w, x, XT, M, N, K, st, sc);
+        }
+    }
+    if (N <= 64 && !forced) {
         const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
         const int tiles64 = (M + 63) / 64;
         if (tiles64 <= cus && 4 * tiles64 >= cus) {
@@ -1311,18 +1336,10 @@ static hipError_t launch_tokens_t(void *y, const uint8_t *w, const uint16_t *x, 
     // Short rows (nb < 16): the register kernel, never split over K (every
     // row is at most 15 super-blocks, dealt to the waves of one workgroup).
     if (t2 * kWaves >= 1024 && wide) {  // (more tokens on as many rows: staged above)
-        gemv_tokens_kernel<XT, YT, 2, kWaves, true>
-            <<<dim3(t2, 1), kWaves * 64, 0, st>>>(y, w, x, M, n_tok, K, nullptr, nb);
-    } else {
-        const int t1 = (M + 15) / 16;
-        if (wide)
-            gemv_tokens_kernel<XT, YT, 1, kWaves, true>
-                <<<t1, kWaves * 64, 0, st>>>(y, w, x, M, n_tok, K, nullptr, nb);
-        else
-            gemv_tokens_kernel<XT, YT, 1, kWaves, false>
-                <<<t1, kWaves * 64, 0, st>>>(y, w, x, M, n_tok, K, nullptr, nb);
+        gemv_tokens_kernel<XT, YT, 2, kWaves, true><<<t2, kWaves * 64, 0, st>>>(y, w, x, M, n_tok, K);
+        return hipGetLastError();
     }
-    return hipGetLastError();
+    return launch_tokens_chunks<XT, YT>(y, w, x, M, n_tok, K, st);
 }
 
 hipError_t launch_gemv_tokens(void *y, int y_dtype, const uint8_t *w, const void *x,

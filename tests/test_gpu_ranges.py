@@ -127,10 +127,11 @@ def test_prefill_attention_split_in_a_graph():
 # 64 row tiles of 64 rows, on 64-row tiles (four groups): groups without
 # super-blocks (K of one to three), uneven parts, K splits, partial row tiles,
 # rows that no vector store covers, the first and last token count of a tile.
-SHORT = [(12, 1, 17, 256), (12, 130, 32, 256), (12, 129, 33, 512), (12, 300, 64, 768), (12, 257, 45, 2048),
-         (12, 64, 20, 11008), (12, 4100, 31, 1280), (12, 4101, 47, 256), (12, 4160, 64, 2816),
-         (13, 130, 17, 512), (13, 131, 50, 2304), (13, 4099, 64, 768), (13, 200, 60, 5120),
-         (14, 1, 64, 256), (14, 130, 32, 768), (14, 133, 33, 2304), (14, 4102, 17, 1280), (14, 60, 64, 11008)]
+SHORT = [(12, 1, 17, 4352), (12, 130, 32, 4608), (12, 4700, 33, 512), (12, 3100, 64, 768), (12, 3075, 45, 2048),
+         (12, 64, 20, 11008), (12, 9217, 17, 256), (12, 4100, 31, 1280), (12, 4101, 47, 256), (12, 4160, 64, 2816),
+         (13, 130, 17, 5376), (13, 1400, 50, 2304), (13, 4099, 64, 768), (13, 200, 60, 5120), (13, 3000, 64, 256),
+         (14, 1, 64, 4352), (14, 9300, 32, 768), (14, 1400, 33, 2304), (14, 6000, 17, 1280), (14, 60, 64, 11008),
+         (14, 2400, 64, 256)]
 
 
 def product_case(t, M, N, K, dt, seed):
@@ -163,6 +164,23 @@ def test_short_prompt_products(t, M, N, K):
     print(f"short prompt type {t} [{M} x {K}] x {N}", flush=True)
     for dt in ("f16", "bf16"):
         case = product_case(t, M, N, K, dt, 7300 + M + N)
+        check_product(capi.gemm, *case, t, M, N, K, dt)
+        check_product(capi.gemm_noalloc, *case, t, M, N, K, dt)
+
+
+# Small matrices, 16-token chunks: the last and first sizes of the rule (576
+# workgroups of up to 8 super-blocks, 256 of up to 16), partial chunks and row
+# tiles, many chunks.
+CHUNKS = [(12, 256, 17, 2048), (12, 255, 500, 512), (12, 1, 1000, 256), (12, 1024, 144, 1024), (12, 1040, 144, 1024),
+          (12, 1024, 64, 4096), (12, 1040, 64, 4096), (13, 130, 200, 2048), (13, 2303, 64, 768), (14, 256, 45, 2048),
+          (14, 100, 333, 1280), (14, 2304, 49, 512), (14, 33, 129, 4096)]
+
+
+@pytest.mark.parametrize("t,M,N,K", CHUNKS)
+def test_small_matrices_in_chunks(t, M, N, K):
+    print(f"chunks type {t} [{M} x {K}] x {N}", flush=True)
+    for dt in ("f16", "bf16"):
+        case = product_case(t, M, N, K, dt, 7450 + M + N)
         check_product(capi.gemm, *case, t, M, N, K, dt)
         check_product(capi.gemm_noalloc, *case, t, M, N, K, dt)
 
