@@ -715,7 +715,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_reduce_kernel(GemmParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// Small batch (2..16 tokens): a workgroup of KW waves owns 16*RT weight rows
+// Small batch (2..16 tokens; chunk blockIdx.y of more): a workgroup of KW waves owns 16*RT weight rows
 // x 16 tokens.  The K super-blocks are dealt to the waves round-robin (wave
 // w: w, w+KW, ...); each wave computes RT 16x16 fragments with
 // v_mfma_f32_16x16x32 (A = 16 weight rows, B = the 16 tokens), so one x
@@ -1148,7 +1148,7 @@ static hipError_t launch_gemm_tm(void *y, const uint8_t *w, const uint16_t *x, i
     // 4096] 18.2 -> 10.2 / 12.8 (10.9 / 14.1), [2048 x 11008] 20.1 -> 13.0 /
     // 16.3, [28672 x 4096] 43 -> 22.4 / 28.3 (25.6 / 36.1 with 64 rows);
     // Q5_K alike, Q6_K 45 tokens [11008 x 2048] 25.5 -> 20.6, [28672 x 4096]
-    // 57.5 -> 47.4.  65 tokens in two tiles are no faster than one of 128.
+    // 57.5 -> 47.4.
     // RXQ4_GEMM_* ask for the larger tiles.
     const Tuning &t = tuning();
     const bool forced = t.gemm_splits || t.gemm_tm || t.gemm_order || t.gemm_mixed || t.gemm_nw;
@@ -1179,6 +1179,23 @@ static hipError_t launch_gemm_tm(void *y, const uint8_t *w, const uint16_t *x, i
         }
         if (N <= 32) return launch_gemm_t<T, XT, YT, 32, 4, 2>(y, w, x, M, N, K, st, sc);
         return launch_gemm_t<T, XT, YT, 64, 4, 2>(y, w, x, M, N, K, st, sc);
+    }
+    // More tokens on matrices whose 64-row, 64-token tiles still fit one round
+    // of the CUs: the same tiles, because 128-token tiles there leave most CUs
+    // idle or pay for K splits, partials and a second launch.  Rows of at most
+    // 12 super-blocks (Q4_K 16: its weights cost less to widen again for each
+    // token tile).  65 / 256 / 512 tokens, us, against the larger tiles:
+    // [2048 x 2048] Q4_K 14.1 / 16.4 / 22.1 -> 10.1 / 12.9 / 12.0, Q6_K 17.0 /
+    // 19.8 / 24.9 -> 12.0 / 14.2 / 17.3; 65 tokens [8192 x 2048] Q4_K 21.4 ->
+    // 12.4, Q5_K 22.8 -> 14.1, [4096 x 4096] Q4_K 18.7 -> 14.9; 128 tokens
+    // [8192 x 4096] Q4_K 23.1 -> 21.4.  Past the rule: [8192 x 4096] at 128
+    // tokens Q5_K 23.5 -> 25.4, Q6_K 26.6 -> 31.3; two rounds, [11008 x 2048]
+    // at 160 Q4_K 25.8 -> 30.8.
+    if (N > 64 && !forced) {
+        const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
+        const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 63) / 64);
+        if (tiles <= cus && K / 256 <= (T == 12 ? 16 : 12))
+            return launch_gemm_t<T, XT, YT, 64, 2, 4>(y, w, x, M, N, K, st, sc);
     }
     if (tm != 128 && tm != 256) {
         const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;

@@ -185,6 +185,23 @@ def test_small_matrices_in_chunks(t, M, N, K):
         check_product(capi.gemm_noalloc, *case, t, M, N, K, dt)
 
 
+# 64-token tiles on more than 64 tokens: the last and first row and token counts
+# of one round (256 tiles), the longest rows of the rule and the next, a last token
+# tile of one token, a last row tile of one row.
+MID = [(12, 8192, 65, 256), (12, 8193, 128, 512), (12, 4097, 130, 2048), (12, 2600, 384, 512), (12, 1025, 193, 4096),
+       (12, 200, 321, 4352), (13, 1100, 450, 768), (13, 2049, 192, 3072), (13, 300, 257, 3328), (14, 8192, 128, 256),
+       (14, 1601, 129, 2304), (14, 500, 640, 3072), (14, 65, 300, 3328)]
+
+
+@pytest.mark.parametrize("t,M,N,K", MID)
+def test_mid_prompt_products(t, M, N, K):
+    print(f"mid prompt type {t} [{M} x {K}] x {N}", flush=True)
+    for dt in ("f16", "bf16"):
+        case = product_case(t, M, N, K, dt, 7600 + M + N)
+        check_product(capi.gemm, *case, t, M, N, K, dt)
+        check_product(capi.gemm_noalloc, *case, t, M, N, K, dt)
+
+
 # Q4_K batches around the row counts from which x is staged in LDS.
 STAGED = [(12, 8192, 5, 768), (12, 8193, 4, 768), (12, 8193, 8, 2048), (12, 5056, 16, 512), (12, 5057, 9, 512),
           (12, 5060, 16, 3840), (12, 9000, 3, 256)]
