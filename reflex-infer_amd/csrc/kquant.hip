@@ -30,7 +30,8 @@
 //   Q6_K: y += d*sc_j * sum((q - 32) x)       (bias 32)
 //   Q5_K: y += d*sc * sum(q x) - dmin*m * sum(x)
 // Rows with 4*K/256 <= 64 slots (K <= 4096, power-of-two block counts) are
-// packed 64/slots rows per wave step; longer rows take one wave per row.
+// packed 64/slots rows per wave step; longer rows take one
+// wave per row, or 8 to 32 lanes of one where that wastes fewer (kq_lanes).
 #include <algorithm>
 #include <type_traits>
 
@@ -1015,8 +1016,8 @@ __global__ __launch_bounds__(256) void kq_tokens_kernel(void *__restrict__ y,
     }
 }
 
-// Small batches (the C ABI sends more than 16 tokens to the GEMM of
-// gemm_q4k.hip): one 16-token fragment per workgroup (grid.y walks the
+// Small batches (more than 16 tokens go to the GEMM of gemm_q4k.hip, which
+// sends small matrices back here, any token count): one 16-token fragment per workgroup (grid.y walks the
 // 16-token chunks), 32 rows when that still gives a workgroup per CU.  With
 // fewer workgroups than four per CU, rows of 20 blocks or more are split over
 // workgroups, a wave keeping at least two blocks (one block after another per

@@ -136,7 +136,7 @@ hipError_t launch_kq_embed(uint16_t *dst, const uint8_t *w, const int32_t *ids, 
 // Tuning overrides from the environment, read once per process (for sweeps;
 // 0 / true = the launchers' defaults):
 //   RXQ4_GEMM_SPLITS, RXQ4_GEMV_WAVES_PER_CU, RXQ4_GEMV_LDS_WAVES_PER_CU,
-//   RXQ4_ATTN_SPLIT (cap on decode chunks), RXQ4_ATTN_MFMA=0 (VALU prefill),
+//   RXQ4_ATTN_SPLIT (cap on attention chunks), RXQ4_ATTN_MFMA=0 (VALU prefill),
 //   RXQ4_MULTI_TOKEN_GEMV=0 (2..4 tokens on the MFMA small-batch kernel),
 //   RXQ4_GEMM_TM=128|256 (the GEMM's token tile),
 //   RXQ4_GEMM_ORDER=1|2 (the GEMM's unit order: row-major | token-major),
