@@ -24,8 +24,14 @@
 //                   ds_read_tr16_b64 of the row-major V), src1 = P^T straight
 //                   from the score registers: k = 8 h + e stands for position
 //                   16 kk + 8 (e / 4) + 4 h + e % 4 in both operands.  P is
-//                   split into fp16 hi + lo (two MFMAs), ~22 bits of the fp32
-//                   probabilities.
+//                   split into fp16 hi + lo (two MFMAs): 22 bits of the fp32
+//                   probabilities down to 2^-35 of the reference point.
+// int8 caches: P holds the V scales, so m follows the maximum of score + log2
+// |scale|; O and l are relative to it all the same.  Scales in P without that ran
+// into fp16's ends: 2000 positions of head_dim 96, error of the split against 64
+// bits at scales around 1e-3 / 1e-4 / 1e-5 2.0e-4 / 2.0e-3 / 2.1e-2, with it 6.5e-8
+// each (an fp16 output's own rounding is 2.0e-4 / 2.2e-4 / 1.1e-3), and NaN from a
+// scale of 4094.
 // Bound: the matrix cores (48 MFMAs of 32 cycles a tile and wave at head_dim
 // 128) and the VALU's exponentials beside them.  32 query rows a wave halve
 // the LDS fragment bytes per MFMA against 16 rows (1 KB per 32 cycles and
@@ -77,7 +83,17 @@ typedef short v4i16 __attribute__((ext_vector_type(4)));
 constexpr int kTile = 64;    // positions per tile
 constexpr int kBlock = 128;  // query rows per workgroup
 constexpr int kMaxChunks = 64;  // KV chunks per block
+// The reference point m of a row's exponentials moves when the row's maximum has
+// outgrown it by 2^kLazy, and P holds 2^kShift times them, up to 2^(kLazy +
+// kShift) = 2^15: fp16's range is used from its top (65504) and the low half of
+// P ends at 2^-24 = 2^-35 of the reference point.
 constexpr float kLazy = 4.0f;
+constexpr float kShift = 11.0f;
+// V scales below 2^kMinScale count as that where the reference point is chosen
+// (what they weigh is 0 in an fp16 output) and those above 2^kMaxScale as that.
+constexpr float kMinScale = -40.0f, kMaxScale = 127.0f;
+// An int8 tile's floats in LDS: K scales, V scales, log2 |V scale|.
+constexpr int kScl = 3 * kTile;
 
 struct PrefillParams {
     uint16_t *out;
@@ -92,6 +108,7 @@ struct PrefillParams {
     int negate;    // scale < 0: q enters negated
 };
 
+typedef const float __attribute__((address_space(1))) *GlobalFloat;
 __device__ const float g_one = 1.0f;  // int8 caches without scales: read with stride 0
 
 __device__ __forceinline__ f32x16 mfma32h(u32x4 a, u32x4 b, f32x16 c) {
@@ -148,7 +165,7 @@ constexpr int tile_bytes() { return kTile * HD * 2; }
 template <int HD, int G>
 constexpr int prefill_lds() {
     return G * 4 * tile_bytes<HD>()      // K, V x 2 buffers
-           + G * 2 * 2 * kTile * 4       // int8 scales
+           + G * 2 * kScl * 4            // int8 scales
            + 2 * 256 * 4;                // (m, l) of the second group
 }
 
@@ -167,8 +184,8 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_kernel(PrefillParams p) 
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r32 = lane & 31, h = lane >> 5;
     uint8_t *const lds = smem + gq * 4 * TB;  // buffer b: K at 2 b TB, V at (2 b + 1) TB
-    float *const scl = reinterpret_cast<float *>(smem + G * 4 * TB) + gq * 4 * kTile;
-    float *const mgl = reinterpret_cast<float *>(smem + G * 4 * TB + G * 16 * kTile);
+    float *const scl = reinterpret_cast<float *>(smem + G * 4 * TB) + gq * 2 * kScl;
+    float *const mgl = reinterpret_cast<float *>(smem + G * 4 * TB + G * 8 * kScl);
 
     // Unit: longest blocks (the latest tokens) first.
     const int kvh = blockIdx.x % p.n_kv;
@@ -195,8 +212,9 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_kernel(PrefillParams p) 
     const int64_t row_stride = (int64_t)p.n_kv * p.hd * esz;
     const uint8_t *kb = static_cast<const uint8_t *>(p.k) + (int64_t)kvh * p.hd * esz;
     const uint8_t *vb = static_cast<const uint8_t *>(p.v) + (int64_t)kvh * p.hd * esz;
-    const float *ksp = p.ks ? p.ks + kvh : &g_one;
-    const float *vsp = p.vs ? p.vs + kvh : &g_one;
+    // (global pointers: a generic load would be waited for with the LDS reads)
+    const GlobalFloat ksp = p.ks ? (GlobalFloat)(p.ks + kvh) : (GlobalFloat)&g_one;
+    const GlobalFloat vsp = p.vs ? (GlobalFloat)(p.vs + kvh) : (GlobalFloat)&g_one;
     const int s_stride = p.ks ? p.n_kv : 0, v_stride = p.vs ? p.n_kv : 0;
     const int n_ch = p.hd >> 3;
 
@@ -239,14 +257,14 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_kernel(PrefillParams p) 
         Chunk c[NC];
         float s;
     };
-    auto load_raw = [&](const uint8_t *base, const float *scales, int stride, int t, Raw &R) {
+    auto load_raw = [&](const uint8_t *base, GlobalFloat scales, int stride, int t, Raw &R) {
         const __amdgpu_buffer_rsrc_t rs = tile_rsrc(base, t * kTile);
 #pragma unroll
         for (int j = 0; j < NC; ++j) {
             if constexpr (I8) R.c[j] = buffer_load8(rs, io[j]);
             else R.c[j] = buffer_load16(rs, io[j]);
         }
-        if (I8 && tid < kTile) R.s = scales[(int64_t)min(t * kTile + tid, pos_end - 1) * stride];
+        if (I8) R.s = scales[(int64_t)min(t * kTile + lane, pos_end - 1) * stride];  // (every wave)
     };
     auto widen = [](Chunk c) {
         if constexpr (I8) {
@@ -260,6 +278,19 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_kernel(PrefillParams p) 
 #pragma unroll
         for (int j = 0; j < NC; ++j) *reinterpret_cast<u32x4 *>(lds + off + place[j]) = widen(R.c[j]);
         if (I8 && tid < kTile) scl[s_off + tid] = R.s;
+    };
+    // log2 |V scale| of the tile's positions, clamped, and a bound of all so far
+    // with a margin, so that it seldom moves (a maximum over the lanes for every
+    // tile costs 3%).  None for the first tile, whose maximum is taken exactly.
+    float lane_log = kMinScale, most_log = kMaxScale;
+    auto store_log = [&](float vs, int s_off, bool first) {
+        if constexpr (I8) {
+            const float lg = fminf(fmaxf(__builtin_amdgcn_logf(fabsf(vs)), kMinScale), kMaxScale);
+            lane_log = fmaxf(lane_log, lg);
+            if (!first && (__builtin_amdgcn_ballot_w64(lane_log > most_log) != 0 || most_log >= kMaxScale))
+                most_log = butterfly_max<64>(lane_log) + 0.125f;
+            if (tid < kTile) scl[s_off + tid] = lg;
+        }
     };
 
     // Lane parts of the fragment addresses: K row 32 pt + r32, chunk
@@ -293,7 +324,7 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_kernel(PrefillParams p) 
                 s[pt] = mfma32h(*reinterpret_cast<const u32x4 *>(kt + ka[ks] + pt * 64 * HD), qf[ks], s[pt]);
         }
         if constexpr (I8) {
-            const float *sk = scl + b * 2 * kTile;
+            const float *sk = scl + b * kScl;
 #pragma unroll
             for (int pt = 0; pt < 2; ++pt)
 #pragma unroll
@@ -310,15 +341,35 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_kernel(PrefillParams p) 
                 for (int i = 0; i < 16; ++i)
                     if (p0 + 32 * pt + 8 * (i >> 2) + 4 * h + (i & 3) > qpos) s[pt][i] = -INFINITY;
         }
+        // the row's largest P in log2 units: the score, with V scales score +
+        // log2 |scale|, at most the largest of each together
         float mx = -INFINITY;
 #pragma unroll
         for (int pt = 0; pt < 2; ++pt)
 #pragma unroll
             for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[pt][i]);
         mx = max_xor_rows<32>(mx) * p.sl2;
+        if constexpr (I8) {
+            const float *sg = scl + b * kScl + 2 * kTile;
+            if (__builtin_amdgcn_ballot_w64(mx + most_log > m + kLazy) != 0) {  // m may have to move: exactly
+                mx = -INFINITY;
+#pragma unroll
+                for (int pt = 0; pt < 2; ++pt)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const f32x4 x = *reinterpret_cast<const f32x4 *>(sg + 32 * pt + 8 * j + 4 * h);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            mx = fmaxf(mx, __builtin_fmaf(s[pt][4 * j + i], p.sl2, x[i]));
+                    }
+                mx = max_xor_rows<32>(mx);
+            } else {
+                mx = -INFINITY;
+            }
+        }
         // m moves when some row's maximum has outgrown it by 2^kLazy (always
-        // at a row's first visible position): e <= 2^kLazy, in range for the
-        // fp16 halves of P, and O and l stay relative to the same m
+        // at a row's first visible position): |P| <= 2^(kLazy + kShift), and O
+        // and l stay relative to the same m
         if (__builtin_amdgcn_ballot_w64(mx > m + kLazy) != 0) {
             const float m_new = fmaxf(m, mx);
             const float corr = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);
@@ -329,12 +380,12 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_kernel(PrefillParams p) 
 #pragma unroll
                 for (int i = 0; i < 16; ++i) o[dt][i] *= corr;
         }
-        const float m_use = m == -INFINITY ? 0.0f : m;  // rows with nothing visible yet: e = 0
+        const float m_use = m == -INFINITY ? 0.0f : m - kShift;  // rows with nothing visible yet: e = 0
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) {
             f32x4 x0, x1;
             if constexpr (I8) {
-                const float *sv = scl + b * 2 * kTile + kTile;
+                const float *sv = scl + b * kScl + kTile;
                 x0 = *reinterpret_cast<const f32x4 *>(sv + 16 * kk + 4 * h);
                 x1 = *reinterpret_cast<const f32x4 *>(sv + 16 * kk + 8 + 4 * h);
             }
@@ -390,13 +441,14 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_kernel(PrefillParams p) 
         load_raw(kb, ksp, s_stride, t, K);
         load_raw(vb, vsp, v_stride, t, V);
     };
-    auto store_tile = [&](int b) {
-        store_raw(K, b * 2 * TB, ik, b * 2 * kTile);
-        store_raw(V, (b * 2 + 1) * TB, iv, b * 2 * kTile + kTile);
+    auto store_tile = [&](int b, bool first) {
+        store_raw(K, b * 2 * TB, ik, b * kScl);
+        store_raw(V, (b * 2 + 1) * TB, iv, b * kScl + kTile);
+        store_log(V.s, b * kScl + 2 * kTile, first);
     };
     if (n_j > 0) {
         load_tile(t_first);
-        store_tile(0);
+        store_tile(0, true);
     }
     for (int j = 0; j < n_it; ++j) {
         wait_lgkmcnt0();
@@ -406,7 +458,7 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_kernel(PrefillParams p) 
         const bool live = j < n_j && t * kTile < wave_end;  // uniform
         if (next) load_tile(t + G);
         if (live) softmax(t, j & 1);
-        if (next) store_tile((j + 1) & 1);
+        if (next) store_tile((j + 1) & 1, false);
         if (live) weigh(j & 1);
     }
     wait_lgkmcnt0();

@@ -98,6 +98,101 @@ def test_prefill_attention_ranges(H, KV, D, N, start, i8):
         assert util.rounded_ok(host16(out).reshape(ref.shape), ref).all(), scale
 
 
+def aligned_inputs(H, KV, D, N, S, height, g, i8):
+    """q, K, V (fp16, or int8 K and V with K scales) whose scores at scale 1 / D
+    are close to height[pos] * a for query rows of a = 0.5 .. 2: every query row
+    and K row is a multiple of one +-1 vector of its KV head, with some noise.
+    V is positive, so that no output is a small difference."""
+    rnd = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    u = torch.sign(rnd(KV, D))
+    a = torch.exp2(torch.rand(N, H, 1, generator=g, device="cuda") * 2 - 1)
+    q = (a * u.repeat_interleave(H // KV, 0) + 0.02 * rnd(N, H, D)).half().view(N, H * D)
+    if not i8:
+        return q, (height.view(-1, 1, 1) * u + 0.02 * rnd(S, KV, D)).half(), (rnd(S, KV, D).abs() + 0.5).half(), None
+    k = (u * 60 + rnd(S, KV, D)).round().clamp(-127, 127).to(torch.int8)
+    v = (rnd(S, KV, D).abs() * 20 + 10).round().clamp(0, 127).to(torch.int8)
+    return q, k, v, (height.view(-1, 1) / 60).expand(S, KV).contiguous()
+
+
+# Where the query rows split over the KV chunks and where they do not, both wave
+# groups, every padded head size.
+DIMS = [(16, 4, 128, 45, 4000), (32, 8, 128, 1100, 0), (4, 2, 80, 70, 500), (8, 2, 64, 40, 3000), (6, 2, 96, 130, 900),
+        (4, 1, 256, 40, 2000)]
+
+
+@pytest.mark.parametrize("i8", [False, True])
+@pytest.mark.parametrize("H,KV,D,N,start", DIMS)
+def test_prefill_attention_rising_scores(H, KV, D, N, start, i8):
+    """Scores that rise along the positions, by more than 2^4 in some tiles, by
+    less in others and differently for each row, and one late key above all:
+    every move of a row's reference point, in walks, wave groups and chunks."""
+    print(f"rising scores H={H} KV={KV} D={D} N={N} start={start} int8={i8}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(7110 + D)
+    S = start + N
+    tile = torch.arange(S, device="cuda") // 64
+    step = torch.tensor([0.0, 3.0, 0.5, -6.0, 4.5, 0.0, 2.0], device="cuda")
+    height = step[tile % 7].masked_fill(torch.arange(S, device="cuda") % 64 != 5, 0.0).cumsum(0)
+    height = height / max(1.0, float(height.max()) / 24)
+    for late in (False, True):
+        if late:
+            height[S * 3 // 4] = float(height.max()) + 9
+        q, k, v, ks = aligned_inputs(H, KV, D, N, S, height, g, i8)
+        vs = torch.rand(S, KV, generator=g, device="cuda") * 0.02 + 0.005 if i8 else None
+        out = torch.full((N, H * D), float("nan"), dtype=torch.float16, device="cuda")
+        capi.attention_prefill_f16(out, q, k, v, H, KV, D, N, start, 1.0 / D, i8, ks, vs)
+        ref = attention64(q, k, v, H, KV, D, N, start, 1.0 / D, ks, vs).cpu().numpy()
+        assert util.rounded_ok(host16(out).reshape(ref.shape), ref).all(), late
+
+
+@pytest.mark.parametrize("H,KV,D,N,start", DIMS)
+def test_prefill_attention_small_probabilities(H, KV, D, N, start):
+    """One position 2^26 above the rest whose V row is 0: what is left is made of
+    probabilities below fp16's smallest."""
+    print(f"small probabilities H={H} KV={KV} D={D} N={N} start={start}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(7120 + D)
+    S = start + N
+    height = torch.zeros(S, device="cuda")
+    height[S // 3] = 26.0 * 0.6931
+    q, k, v, _ = aligned_inputs(H, KV, D, N, S, height, g, False)
+    q = torch.sign(q)  # every row's a is 1
+    v *= 64
+    v[S // 3] = 0
+    out = torch.full((N, H * D), float("nan"), dtype=torch.float16, device="cuda")
+    capi.attention_prefill_f16(out, q, k, v, H, KV, D, N, start, 1.0 / D)
+    ref = attention64(q, k, v, H, KV, D, N, start, 1.0 / D).cpu().numpy()
+    sees = slice(max(0, S // 3 - start), N)
+    # 2^-11: half a unit of an fp16 output and as much again for the sums
+    assert util.rounded_ok(host16(out).reshape(ref.shape)[sees], ref[sees], delta=2.0 ** -12).all()
+
+
+@pytest.mark.parametrize("size", ["1e-6", "1e-4", "3e4", "mixed", "zeros"])
+@pytest.mark.parametrize("H,KV,D,N,start", DIMS)
+def test_prefill_attention_v_scales(H, KV, D, N, start, size):
+    """int8 caches whose V scales are far from 1, with one position above the
+    rest by up to 2^24: the probabilities keep their precision and, where it is
+    below 2^4 and the reference point of the exponentials stays, their range."""
+    print(f"V scales {size} H={H} KV={KV} D={D} N={N} start={start}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(7130 + D)
+    S = start + N
+    height = torch.rand(S, generator=g, device="cuda")
+    height[S // 3] += (1.4 if size == "3e4" else 12) * 0.6931
+    q, k, v, ks = aligned_inputs(H, KV, D, N, S, height, g, True)
+    vs = torch.rand(S, KV, generator=g, device="cuda") + 0.5
+    if size == "mixed":  # over 2^16 in every tile
+        vs *= torch.exp2(torch.rand(S, KV, generator=g, device="cuda") * 16 - 14)
+        vs *= torch.sign(torch.rand(S, KV, generator=g, device="cuda") - 0.05)
+    elif size == "zeros":
+        vs[: S // 2] = 0
+    else:
+        vs *= float(size)
+        if size == "3e4":
+            v = v % 2  # the outputs are fp16
+    out = torch.full((N, H * D), float("nan"), dtype=torch.float16, device="cuda")
+    capi.attention_prefill_f16(out, q, k, v, H, KV, D, N, start, 1.0 / D, True, ks, vs)
+    ref = attention64(q, k, v, H, KV, D, N, start, 1.0 / D, ks, vs).cpu().numpy()
+    assert util.rounded_ok(host16(out).reshape(ref.shape), ref).all()
+
+
 def test_prefill_attention_split_in_a_graph():
     """A split prefill captured on a stream without a workspace, replayed with
     other work between: every replay equals the eager result."""
