@@ -172,7 +172,11 @@ int rxq4_attention_decode_f16(void *out, const void *q, const void *k_cache,
                               const float *v_scales, void *stream);
 
 /* Prefill: N query tokens q[N x n_heads x head_dim]; token t attends to
- * positions [0, start_pos + t + 1) of the caches (causal).
+ * positions [0, start_pos + t + 1) of the caches (causal).  What the caches
+ * hold past a token's last position does not reach its row, infinities and NaN
+ * included, with one exception: at head_dim 64 and 128, where the launcher picks
+ * the kernel for short prompts, an infinity or NaN in V or v_scales may reach
+ * the earlier tokens of its 64-position tile.
  * Replaces kernels::flash_attention_prefill_batched (reference
  * attention.cu:432-448, 180-290). */
 int rxq4_attention_prefill_f16(void *out, const void *q, const void *k_cache,

@@ -116,6 +116,33 @@ __device__ __forceinline__ f32x16 mfma32h(u32x4 a, u32x4 b, f32x16 c) {
                                                   __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
 
+// Infinities and NaN among N x 8 fp16: whether there are any (times 0 they are
+// NaN), and zeros in their place (a half with all exponent bits set carries into
+// its top bit).
+template <int N>
+__device__ __forceinline__ bool not_finite16(const u32x4 *x) {
+    f16x2 sum[4] = {};
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t v = x[j][i];  // (a bit cast of the vector's element itself takes element 0)
+            sum[i] = __builtin_elementwise_fma(__builtin_bit_cast(f16x2, v), f16x2{0, 0}, sum[i]);
+        }
+    const f16x2 all = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+    return !(all.x == 0) || !(all.y == 0);
+}
+template <int N>
+__device__ __forceinline__ void zero_not_finite16(u32x4 *x) {
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t all = (((x[j][i] & 0x7C007C00u) + 0x04000400u) >> 15) & 0x00010001u;
+            x[j][i] &= ~(all * 0xFFFFu);
+        }
+}
+
 // Token and head of query row row0 + r (r < 32), from the uniform division of
 // row0: the quotient of rem0 + r < group + 32 by the group from a reciprocal
 // ((x + 0.5) / group is at least 0.5 / group from an integer, far more than
@@ -166,7 +193,8 @@ template <int HD, int G>
 constexpr int prefill_lds() {
     return G * 4 * tile_bytes<HD>()      // K, V x 2 buffers
            + G * 2 * kScl * 4            // int8 scales
-           + 2 * 256 * 4;                // (m, l) of the second group
+           + 2 * 256 * 4                 // (m, l) of the second group
+           + G * 4 * 4;                  // a wave's flag: V not finite
 }
 
 template <int HD, bool I8, int G>
@@ -186,6 +214,7 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_kernel(PrefillParams p) 
     uint8_t *const lds = smem + gq * 4 * TB;  // buffer b: K at 2 b TB, V at (2 b + 1) TB
     float *const scl = reinterpret_cast<float *>(smem + G * 4 * TB) + gq * 2 * kScl;
     float *const mgl = reinterpret_cast<float *>(smem + G * 4 * TB + G * 8 * kScl);
+    int *const bad_v = reinterpret_cast<int *>(mgl + 512) + gq * 4;
 
     // Unit: longest blocks (the latest tokens) first.
     const int kvh = blockIdx.x % p.n_kv;
@@ -217,6 +246,7 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_kernel(PrefillParams p) 
     const GlobalFloat vsp = p.vs ? (GlobalFloat)(p.vs + kvh) : (GlobalFloat)&g_one;
     const int s_stride = p.ks ? p.n_kv : 0, v_stride = p.vs ? p.n_kv : 0;
     const int n_ch = p.hd >> 3;
+    const int blk_first = p.start + block * kBlock / p.group;  // first query position of the block
 
     // Q^T fragments: dims 16 ks + 8 h .. + 7 of the row (zeros past hd).
     u32x4 qf[KS];
@@ -233,15 +263,25 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_kernel(PrefillParams p) 
     }
 
     // The thread's chunks of a tile: source offset within the tile's rows
-    // (past the resource for dims past head_dim: zeros), LDS offsets.
-    int io[NC], ik[NC], iv[NC];
+    // (past the resource for dims past head_dim: zeros), LDS offsets.  Where a row
+    // divides the 256 chunks, chunk j is kRows rows down and the places in a K row
+    // repeat every kPerK chunks: only what differs is kept.
+    constexpr bool kEven = 256 % CH == 0;
+    constexpr int kRows = 256 / CH, kPer = kEven ? 1 : NC, kPerK = kEven && kRows % 16 ? 16 / kRows : kPer;
+    static_assert(!kEven || kRows % 4 == 0, "the places in a V row repeat");
+    int io[kPer], ik[kPerK], iv[kPer];
 #pragma unroll
-    for (int j = 0; j < NC; ++j) {
+    for (int j = 0; j < kPerK; ++j) {
         const int id = tid + 256 * j, pr = id / CH, c = id % CH;
-        io[j] = c < n_ch ? (int)(pr * row_stride) + 8 * esz * c : 0x7FFFFFF0;
         ik[j] = pr * HD * 2 + 16 * k_pos<HD>(pr, c);
+        if (j >= kPer) continue;
+        io[j] = c < n_ch ? (int)(pr * row_stride) + 8 * esz * c : 0x7FFFFFF0;
         iv[j] = pr * HD * 2 + 16 * v_pos<HD>(pr, c);
     }
+    const int io_step = tid % CH < n_ch ? kRows * (int)row_stride : 0;
+    auto chunk_src = [&](int j) { return kEven ? io[0] + j * io_step : io[j % kPer]; };
+    auto chunk_k = [&](int j) { return ik[j % kPerK] + (kEven ? j / kPerK * kPerK * kRows * HD * 2 : 0); };
+    auto chunk_v = [&](int j) { return kEven ? iv[0] + j * kRows * HD * 2 : iv[j % kPer]; };
     // resources over a tile's visible rows (rows past them read zeros); the
     // base and bound are wave-uniform
     auto tile_rsrc = [&](const uint8_t *base, int p0) {
@@ -261,8 +301,8 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_kernel(PrefillParams p) 
         const __amdgpu_buffer_rsrc_t rs = tile_rsrc(base, t * kTile);
 #pragma unroll
         for (int j = 0; j < NC; ++j) {
-            if constexpr (I8) R.c[j] = buffer_load8(rs, io[j]);
-            else R.c[j] = buffer_load16(rs, io[j]);
+            if constexpr (I8) R.c[j] = buffer_load8(rs, chunk_src(j));
+            else R.c[j] = buffer_load16(rs, chunk_src(j));
         }
         if (I8) R.s = scales[(int64_t)min(t * kTile + lane, pos_end - 1) * stride];  // (every wave)
     };
@@ -274,23 +314,44 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_kernel(PrefillParams p) 
             return c;
         }
     };
-    auto store_raw = [&](const Raw &R, int off, const int *place, int s_off) {
+    auto store_raw = [&](const Raw &R, int off, auto place, int s_off) {
 #pragma unroll
-        for (int j = 0; j < NC; ++j) *reinterpret_cast<u32x4 *>(lds + off + place[j]) = widen(R.c[j]);
+        for (int j = 0; j < NC; ++j) *reinterpret_cast<u32x4 *>(lds + off + place(j)) = widen(R.c[j]);
         if (I8 && tid < kTile) scl[s_off + tid] = R.s;
     };
-    // log2 |V scale| of the tile's positions, clamped, and a bound of all so far
-    // with a margin, so that it seldom moves (a maximum over the lanes for every
-    // tile costs 3%).  None for the first tile, whose maximum is taken exactly.
-    float lane_log = kMinScale, most_log = kMaxScale;
+    // log2 |V scale| of the tile's positions, clamped, and a bound of theirs that
+    // seldom moves (a maximum over the lanes for every tile costs 3%).  None for
+    // the first tile, where the row's maximum is taken exactly in any case.
+    float most_log = kMaxScale;
     auto store_log = [&](float vs, int s_off, bool first) {
         if constexpr (I8) {
             const float lg = fminf(fmaxf(__builtin_amdgcn_logf(fabsf(vs)), kMinScale), kMaxScale);
-            lane_log = fmaxf(lane_log, lg);
-            if (!first && (__builtin_amdgcn_ballot_w64(lane_log > most_log) != 0 || most_log >= kMaxScale))
-                most_log = butterfly_max<64>(lane_log) + 0.125f;
+            if (!first && (__builtin_amdgcn_ballot_w64(lg > most_log) != 0 || most_log >= kMaxScale))
+                most_log = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(
+                               int, butterfly_max<64>(lg) + 0.125f)));
             if (tid < kTile) scl[s_off + tid] = lg;
         }
+    };
+
+    // Positions that some row of the block does not see: a zero probability does
+    // not stop an infinity or NaN there in the P.V products.  On the tiles that
+    // hold such positions those V values (int8: V scales) are staged again as
+    // zeros, and the rows that see them get them at the end.  (Looked over after
+    // their LDS writes have gone out: 300 tokens after 700 at head_dim 96 15.5 ->
+    // 15.8 us, 2048 from 0 at 128 unchanged; rows of a clean cache bit for bit.)
+    if (lane == 0) bad_v[w] = 0;  // the wave's flag: some of its staging
+    auto look_over = [&](Raw &R, int t, int off, int s_off) {
+        if (t * kTile + kTile - 1 <= blk_first) return;  // uniform
+        if constexpr (I8) {
+            const bool bad = !(fabsf(R.s) < INFINITY);
+            if (__builtin_amdgcn_ballot_w64(bad) == 0) return;
+            if (bad && tid < kTile) scl[s_off + tid] = 0.0f;
+        } else {
+            if (__builtin_amdgcn_ballot_w64(not_finite16<NC>(R.c)) == 0) return;
+            zero_not_finite16<NC>(R.c);
+            store_raw(R, off, chunk_v, s_off);
+        }
+        if (lane == 0) bad_v[w] = 1;
     };
 
     // Lane parts of the fragment addresses: K row 32 pt + r32, chunk
@@ -367,11 +428,12 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_kernel(PrefillParams p) 
                 mx = -INFINITY;
             }
         }
-        // m moves when some row's maximum has outgrown it by 2^kLazy (always
+        // m moves when the row's maximum has outgrown it by 2^kLazy (always
         // at a row's first visible position): |P| <= 2^(kLazy + kShift), and O
         // and l stay relative to the same m
         if (__builtin_amdgcn_ballot_w64(mx > m + kLazy) != 0) {
-            const float m_new = fmaxf(m, mx);
+            // (each row's by its own rule: no row depends on what others see)
+            const float m_new = mx > m + kLazy ? mx : m;
             const float corr = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);
             m = m_new;
             l *= corr;
@@ -441,14 +503,15 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_kernel(PrefillParams p) 
         load_raw(kb, ksp, s_stride, t, K);
         load_raw(vb, vsp, v_stride, t, V);
     };
-    auto store_tile = [&](int b, bool first) {
-        store_raw(K, b * 2 * TB, ik, b * kScl);
-        store_raw(V, (b * 2 + 1) * TB, iv, b * kScl + kTile);
+    auto store_tile = [&](int t, int b, bool first) {
+        store_raw(K, b * 2 * TB, chunk_k, b * kScl);
+        store_raw(V, (b * 2 + 1) * TB, chunk_v, b * kScl + kTile);
         store_log(V.s, b * kScl + 2 * kTile, first);
+        look_over(V, t, (b * 2 + 1) * TB, b * kScl + kTile);
     };
     if (n_j > 0) {
         load_tile(t_first);
-        store_tile(0, true);
+        store_tile(t_first, 0, true);
     }
     for (int j = 0; j < n_it; ++j) {
         wait_lgkmcnt0();
@@ -458,11 +521,35 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_kernel(PrefillParams p) 
         const bool live = j < n_j && t * kTile < wave_end;  // uniform
         if (next) load_tile(t + G);
         if (live) softmax(t, j & 1);
-        if (next) store_tile((j + 1) & 1, false);
+        if (next) store_tile(t + G, (j + 1) & 1, false);
         if (live) weigh(j & 1);
     }
     wait_lgkmcnt0();
     lds_barrier();
+    if (__builtin_amdgcn_readfirstlane(bad_v[0] | bad_v[1] | bad_v[2] | bad_v[3]) != 0) {
+        for (int t = max(t_beg, (blk_first + 1) / kTile); t < t_end; ++t) {
+            if ((t - t_beg) % G != gq) continue;
+            for (int pos = t * kTile; pos < min(wave_end, t * kTile + kTile); ++pos) {
+                const uint8_t *row = vb + pos * row_stride + 4 * esz * h;
+                const float vs = I8 ? vsp[(int64_t)pos * v_stride] : 1.0f;
+                if (pos > qpos || (I8 && fabsf(vs) < INFINITY)) continue;
+                int n = n_ch;
+                asm volatile("" : "+s"(n));  // (compared here, not kept as CH conditions)
+#pragma unroll
+                for (int c = 0; c < CH; ++c) {
+                    if (c >= n) continue;  // uniform
+                    const u32x2 x = I8 ? u32x2{*reinterpret_cast<const uint32_t *>(row + 8 * c), 0u}
+                                       : *reinterpret_cast<const u32x2 *>(row + 16 * c);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float v = I8 ? vs * (float)(int8_t)(x.x >> (8 * i))
+                                           : f16_bits_to_f32((i < 2 ? x.x : x.y) >> (16 * (i & 1)) & 0xFFFFu);
+                        if (!(fabsf(v) < INFINITY)) o[c / 4][4 * (c % 4) + i] += v;
+                    }
+                }
+            }
+        }
+    }
 
     // Merge: the second group hands (O, m, l) over through its own buffers.
     l = sum_xor_rows<32>(l);

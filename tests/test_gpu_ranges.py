@@ -193,6 +193,50 @@ def test_prefill_attention_v_scales(H, KV, D, N, start, size):
     assert util.rounded_ok(host16(out).reshape(ref.shape), ref).all()
 
 
+@pytest.mark.parametrize("what", ["nan", "inf", "-inf", "k", "scale", "k scale"])
+@pytest.mark.parametrize("H,KV,D,N,start", DIMS + [(2, 2, 80, 64, 64), (5, 1, 144, 31, 0), (4, 4, 48, 300, 1),
+                                                  (32, 8, 128, 45, 8000)])
+def test_prefill_attention_is_causal(H, KV, D, N, start, what):
+    """Infinities and NaN in the caches reach the tokens that see them and no
+    other: the earlier tokens' rows (and dims) are those of a clean cache."""
+    print(f"causal {what} H={H} KV={KV} D={D} N={N} start={start}", flush=True)
+    i8 = "scale" in what
+    g = torch.Generator(device="cuda").manual_seed(7140 + D + N)
+    rnd = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    S = start + N
+    q, scale = rnd(N, H * D).half(), D ** -0.5
+    if i8:
+        k, v = (rnd(S, KV, D).mul(40).round().clamp(-127, 127).to(torch.int8) for _ in range(2))
+        ks, vs = (rnd(S, KV).abs() * 0.01 + 0.02 for _ in range(2))
+    else:
+        k, v, ks, vs = rnd(S, KV, D).half(), rnd(S, KV, D).half(), None, None
+    clean = torch.empty((N, H * D), dtype=torch.float16, device="cuda")
+    capi.attention_prefill_f16(clean, q, k, v, H, KV, D, N, start, scale, i8, ks, vs)
+    for token in sorted({0, 1, N // 2, N - 2, N - 1} & set(range(N))):
+        p = start + token
+        bk, bv, bks, bvs = (None if t is None else t.clone() for t in (k, v, ks, vs))
+        dims = slice(0, D)
+        if what == "k":
+            bk[p, 0, D // 2] = float("nan")
+        elif what == "scale":
+            bvs[p, 0] = float("nan")
+            bvs[p + 1:, 0] = float("inf")
+        elif what == "k scale":
+            bks[p, 0] = float("nan")
+        else:
+            dims = slice(3, 6)
+            bv[p, 0, dims] = float(what)
+        out = torch.full_like(clean, float("nan"))
+        capi.attention_prefill_f16(out, q, bk, bv, H, KV, D, N, start, scale, i8, bks, bvs)
+        o, c = out.view(N, H, D), clean.view(N, H, D)
+        assert torch.equal(o[:token], c[:token])
+        assert torch.equal(o[:, H // KV:], c[:, H // KV:])  # the other KV heads
+        hit = o[token:, : H // KV, dims]
+        assert not torch.isfinite(hit).any()
+        rest = [d for d in range(D) if not dims.start <= d < dims.stop]
+        assert torch.equal(o[token:, : H // KV, rest], c[token:, : H // KV, rest])
+
+
 def test_prefill_attention_split_in_a_graph():
     """A split prefill captured on a stream without a workspace, replayed with
     other work between: every replay equals the eager result."""
