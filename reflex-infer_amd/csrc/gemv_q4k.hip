@@ -995,7 +995,9 @@ __global__ __launch_bounds__(64 * kLdsStreamWaves) void gemv_lds_stream_kernel(G
 // kernels below (graph replay): [27648 x 5120] 26.1 -> 18.3 us (4.4 TB/s),
 // [17920 x 1536] 10.1 -> 6.7, [37888 x 3584] 22.4 -> 17.5, [5120 x 5120] 8.8 ->
 // 6.6, [4096 x 14336] 11.6 -> 9.3, [16384 x 3072] 12.0 -> 8.2, [1536 x 1536]
-// 3.8 -> 3.2.
+// 3.8 -> 3.2.  With a residual, against fetching it where a row ends: [5120 x
+// 5120] 6.9 -> 6.4, [6144 x 3584] 6.2 -> 5.6, [17920 x 3584] 12.5 -> 10.3, [13824
+// x 11008] 21.4 -> 19.5 (whole waves 8.2, 5.6, 10.6, 19.0).
 template <int EPI, int U, int NT, int LPR>
 __global__ __launch_bounds__(256) void gemv_rows_kernel(GemvParams p) {
     constexpr int RPG = 64 / LPR;
@@ -1052,6 +1054,13 @@ __global__ __launch_bounds__(256) void gemv_rows_kernel(GemvParams p) {
     u32x4 xraw[NT][8];
 #pragma unroll
     for (int tk = 0; tk < NT; ++tk) load_x_raw(p.x + (int64_t)tk * K, s_load >> 2, s_load & 3, xraw[tk]);
+    // The residuals of the wave's first 64 rows, a row a lane, ahead of the
+    // weights: fetched where a row ends, they would wait for the batches in
+    // flight (vector loads complete in order).  A row group's residuals are
+    // taken out of the lanes at the end of the group before it.
+    uint32_t res = 0, rres = 0;
+    auto load_res = [&](int g) { return (uint32_t)rg.res[min(g * RPG + lane, last)]; };
+    if (EPI == kEpiAdd) res = load_res(g0);
     __builtin_amdgcn_sched_barrier(0);
     Batch<U> A, B;
     load(A);
@@ -1076,6 +1085,7 @@ __global__ __launch_bounds__(256) void gemv_rows_kernel(GemvParams p) {
     float acc[NT];
 #pragma unroll
     for (int tk = 0; tk < NT; ++tk) acc[tk] = 0.0f;
+    if (EPI == kEpiAdd) rres = (uint32_t)__shfl((int)res, sub);
     int cp_item = 0, cp_g = g0, cp_j = 0;
     auto compute = [&](const Batch<U> &bt) {
 #pragma unroll
@@ -1112,16 +1122,22 @@ __global__ __launch_bounds__(256) void gemv_rows_kernel(GemvParams p) {
                 if (++cp_j == J) {
                     const int row = cp_g * RPG + sub;
                     const bool mine = sl == LPR - 1 && row <= last;
-                    uint32_t res = 0;
-                    if (EPI == kEpiAdd) res = rg.res[min(row, last)];
 #pragma unroll
                     for (int tk = 0; tk < NT; ++tk) {
                         const float total = lane_group_sum<LPR>(acc[tk]);
-                        if (mine) store_row<EPI>(rg, row, total, res, (int64_t)tk * p.y_stride);
+                        if (mine) store_row<EPI>(rg, row, total, rres, (int64_t)tk * p.y_stride);
                         acc[tk] = 0.0f;
                     }
                     cp_j = 0;
                     ++cp_g;
+                    if (EPI == kEpiAdd) {
+                        const int at = (cp_g - g0) * RPG & 63;
+                        if (at == 0) {  // once in 64 rows
+                            res = load_res(cp_g);
+                            asm volatile("" : "+v"(res));  // waited for here, not where it is used
+                        }
+                        rres = (uint32_t)__shfl((int)res, at + sub);
+                    }
                 }
             }
         }
@@ -1266,11 +1282,16 @@ static hipError_t launch_reg(const GemvParams &p, int grid, hipStream_t st) {
 // Ties go to more rows a wave (fewer sums: [8192 x 8192], 16 items either way,
 // 9.7 us with 8 lanes, 10.6 with 64), but to the whole wave where it takes at
 // most two rows (the streamed kernel's one-row waves, two a SIMD: down [2048 x
-// 11008] 5.5-5.9 against 5.7 us with 32 lanes).  Other items against times, 8 /
-// 16 / 32 lanes: [5120 x 13824] 27 / 28 / 21 (64 lanes: 20), 13.2 / 13.6 / 11.6
-// (11.4) us; [4096 x 14336] 28 / 14 / 14, 13.0 / 9.3 / 9.7; [1536 x 8960] 18 /
-// 9 / 5, 8.5 / 6.0 / 4.8.  Rows and length alone decide, so every token count
-// sums a row in the same order.
+// 11008] 5.5-5.9 against 5.7 us with 32 lanes).  The streamed kernel's own waves,
+// eight a CU, have fewer items than that at ties, and it is the slower one there
+// all the same (with a residual, 64 / 16 lanes: [2304 x 2304] 4.05 / 3.67 us, [3072 x
+// 3072] 4.32 / 3.66, [4096 x 3328] 4.62 / 4.32, [3072 x 8960] 8.22 / 6.22); ties go
+// the wrong way only from 10240 rows of 11008 on, with a residual by 1-3% ([13824 x
+// 11008] 19.0 / 19.5 with 32 lanes), without one 4% the right way.  Other items
+// against times, 8 / 16 / 32 lanes: [5120 x 13824] 27 / 28 / 21 (64 lanes: 20),
+// 13.2 / 13.6 / 11.6 (11.4) us; [4096 x 14336] 28 / 14 / 14, 13.0 / 9.3 / 9.7;
+// [1536 x 8960] 18 / 9 / 5, 8.5 / 6.0 / 4.8.  Rows and length alone decide, so
+// every token count sums a row in the same order.
 static int row_lanes(int64_t rows, int nb, int cus) {
     const int64_t waves = 4 * (int64_t)cus;
     int best = 64;

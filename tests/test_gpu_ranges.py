@@ -375,10 +375,11 @@ def test_kquant_batches_split_and_large(t, M, N, K):
 # --------------------------------------------------- decode GEMV, row groups
 # 8, 16 and 32 lanes a row: partial last groups of rows, steps past a row's
 # slots (a multiple of 4 only), several groups a wave, ranges of a pair and a
-# triple ending inside a group, 1 to 4 tokens, the residual in place.
+# triple ending inside a group, 1 to 4 tokens, the residual in place (70001 rows:
+# more than 64 of them a wave).
 ROWS = [((5120,), 5120), ((27649,), 1280), ((17919,), 1536), ((1537,), 1536), ((1536,), 8960), ((4099,), 3584),
         ((2047,), 3072), ((13823, 13825), 768), ((5121, 1, 1023), 5120), ((7, 9, 3), 2816), ((1,), 1792),
-        ((37890,), 3584), ((4097,), 14336), ((3,), 65280)]
+        ((37890,), 3584), ((4097,), 14336), ((3,), 65280), ((70001,), 768)]
 
 
 @pytest.mark.parametrize("rows,K", ROWS)
