@@ -461,7 +461,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnParams p) {
 // Causal: query row (t, h) sees positions [0, start + t]; rows of a tile
 // past that get probability 0 (rows with nothing visible yet keep m = -inf).
 // This kernel serves prompts of at most one workgroup per CU and few tiles (see
-// rows16_preferred); attn_prefill.hip the rest.
+// rows16_us); attn_prefill.hip the rest.
 template <int HD, int HB, bool I8>
 __global__ __launch_bounds__(512) void attn_prefill_mfma(AttnParams p, int start, int n_tok) {
     constexpr int G = 2;               // wave groups
@@ -1026,20 +1026,53 @@ static int64_t rows16_grid(int n_kv, int group, int n_tok) {
     return (int64_t)n_kv * (group / hb) * (((int64_t)n_tok + tpb - 1) / tpb);
 }
 
-// Whether attn_prefill_mfma (64 query rows a workgroup, never split) is the
-// faster one: with one round of workgroups it takes 5.0 + 1.08 us a tile at
-// head_dim 128 (3.8 + 0.78 at 64), its shorter chain against the 128-row
-// kernel's reuse and splits.  Measured, 32 / 8 heads of 128, this kernel
-// against the other: 8 tokens 6.4 / 7.2 us, 200 9.9 / 11.2, 512 14.7 / 17.5;
-// past one round 640 tokens 21.2 / 19.7, 1000 34.7 / 29, 2048 104 / 68; after
-// cached positions 45 + 400 12.5 / 13.4, 45 + 800 19.4 / 14.7, 45 + 8000
-// 134 / 27.
-static bool rows16_preferred(int n_heads, int n_kv, int head_dim, int n_tok, int start, int cus) {
-    if (head_dim != 64 && head_dim != 128) return false;
-    if (rows16_grid(n_kv, n_heads / n_kv, n_tok) > cus) return false;
+// Launch models, microseconds, of the two kernels that walk the positions unsplit,
+// against plan_prefill_attention's of the 128-row kernel.
+
+// The mean of the tokens' visible tiles.
+static double mean_tiles(int n_tok, int start) {
+    const double tiles = (start + n_tok + kAttnTile - 1) / kAttnTile;
+    return std::min(tiles, std::max(1.0, (start + 0.5 * (n_tok + 1)) / kAttnTile + 0.5));
+}
+
+// Head sizes 64 and 128: attn_prefill_mfma (64 query rows a workgroup) within one
+// round of workgroups, its shorter chain against the other's reuse and splits.
+// Measured, 32 / 8 heads of 128, this kernel / the other: 3 tokens 5.5 / 6.7 us, 200
+// 8.8 / 10.9, 512 13.3 / 16.6; past one round 1000 tokens 34.7 / 29; after cached
+// positions 45 + 200 8.8 / 11.4, 45 + 400 11.9 / 13.1, 45 + 700 16.6 / 14.0; 8 / 2
+// heads, 1411 tokens 25.7 / 27.3; int8 200 10.7 / 12.4, 14 / 2 heads 100 + 300 15.1 /
+// 13.5.
+static double rows16_us(int n_heads, int n_kv, int head_dim, int n_tok, int start, int kv_int8, int cus) {
+    if (rows16_grid(n_kv, n_heads / n_kv, n_tok) > cus) return INFINITY;
     const int tiles = (start + n_tok + kAttnTile - 1) / kAttnTile;
-    const double us = head_dim == 64 ? 3.8 + 0.78 * tiles : 5.0 + 1.08 * tiles;
-    return us <= prefill_attention_us(n_heads, n_kv, head_dim, n_tok, start);
+    const double t = 0.8 * tiles + 0.2 * mean_tiles(n_tok, start);
+    if (head_dim == 64) return kv_int8 ? 4.6 + 0.85 * t : 3.4 + 0.72 * t;
+    return kv_int8 ? 6.2 + 1.25 * t : 4.6 + 1.04 * t;
+}
+
+// Query heads of a VALU workgroup: q sits in registers, 8 heads up to 128 dims, 4
+// beyond.
+static int valu_heads(int group, int head_dim) {
+    return std::min(group, head_dim > 128 ? kAttnMaxHeads / 2 : kAttnMaxHeads);
+}
+
+// Other head sizes: the VALU kernel (a workgroup per token and head group), whose
+// tile costs by its heads.  Measured, this kernel / the other: 32 / 8 heads of 80, 3
+// tokens 4.9 / 6.0, 16 after 40 4.9 / 6.4, 3 after 200 12.1 / 8.7, 68 11.1 / 6.6; 4 / 4
+// heads of 96, 68 tokens 5.5 / 7.2, 3 after 200 7.6 / 8.5, 200 12.3 / 9.4; 5 / 1 heads
+// of 256, 16 after 40 6.4 / 10.3, 68 10.2 / 13.4, 68 after 200 19.6 / 13.7; int8 20
+// after 100, 32 / 8 of 256, 12.2 / 13.9.
+static double valu_us(int n_heads, int n_kv, int head_dim, int n_tok, int start, int kv_int8, int cus) {
+    const bool wide = head_dim > 128;
+    const int group = n_heads / n_kv, hpw = valu_heads(group, head_dim);
+    const double per_tile = wide ? (hpw == 1 ? 1.45 : hpw == 2 ? 2.1 : 3.3)
+                                 : (hpw == 1 ? 1.06 : hpw == 2 ? 1.55 : hpw <= 4 ? 2.35 : 3.72);
+    const double tile = kv_int8 ? 1.2 * per_tile : per_tile;
+    const int tiles = (start + n_tok + kAttnTile - 1) / kAttnTile;
+    const int64_t wgs = (int64_t)n_kv * ((group + hpw - 1) / hpw) * n_tok;
+    const int64_t rounds = (wgs + cus - 1) / cus;
+    const double one = (wide || hpw <= 2 ? 3.1 : 2.6) + tile * tiles;
+    return std::max(one, 2.0 + rounds * ((wide ? 2.0 : 0.8) + tile * mean_tiles(n_tok, start)));
 }
 
 template <int HD, bool I8>
@@ -1073,13 +1106,18 @@ hipError_t launch_attention(uint16_t *out, const uint16_t *q, const void *k, con
                             int head_dim, int n_tok, int seq0, float scale, int kv_int8,
                             hipStream_t st) {
     const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
-    const bool rows16 = n_tok > 1 && tuning().attn_mfma &&
-                        rows16_preferred(n_heads, n_kv, head_dim, n_tok, seq0 - 1, cus);
-    if (n_tok > 1 && tuning().attn_mfma && !rows16) {
-        // callers' limit for the head sizes that had a grid row per token
-        if (head_dim != 64 && head_dim != 128 && n_tok > 65535) return hipErrorInvalidValue;
-        return launch_prefill_attention(out, q, k, v, ks, vs, n_heads, n_kv, head_dim, n_tok, seq0 - 1,
-                                        scale, kv_int8, st);
+    const bool prefill = n_tok > 1 && tuning().attn_mfma;
+    const bool has16 = head_dim == 64 || head_dim == 128;
+    if (prefill) {
+        // callers' limit for the head sizes that may take a grid row per token
+        if (!has16 && n_tok > 65535) return hipErrorInvalidValue;
+        const int start = seq0 - 1;
+        const PrefillPlan plan = plan_prefill_attention(n_heads, n_kv, head_dim, n_tok, start, kv_int8);
+        const double other = has16 ? rows16_us(n_heads, n_kv, head_dim, n_tok, start, kv_int8, cus)
+                                   : 1.03 * valu_us(n_heads, n_kv, head_dim, n_tok, start, kv_int8, cus);
+        if (other > plan.us)
+            return launch_prefill_attention(out, q, k, v, ks, vs, n_heads, n_kv, head_dim, n_tok, start,
+                                            scale, kv_int8, plan, st);
     }
     AttnParams p{};
     p.out = out;
@@ -1092,9 +1130,7 @@ hipError_t launch_attention(uint16_t *out, const uint16_t *q, const void *k, con
     p.n_kv = n_kv;
     p.head_dim = head_dim;
     p.group = n_heads / n_kv;
-    // q of the workgroup's heads sits in registers: 8 heads up to 128 dims,
-    // 4 beyond.
-    p.hpw = std::min(p.group, head_dim > 128 ? kAttnMaxHeads / 2 : kAttnMaxHeads);
+    p.hpw = valu_heads(p.group, head_dim);
     p.n_hg = (p.group + p.hpw - 1) / p.hpw;
     p.seq0 = seq0;
     p.scale = scale;
@@ -1126,7 +1162,7 @@ hipError_t launch_attention(uint16_t *out, const uint16_t *q, const void *k, con
             if (e != hipSuccess) return e;
         }
     }
-    if (rows16) {
+    if (prefill && has16) {
         if (head_dim == 64) {
             if (kv_int8) launch_prefill_hd<64, true>(p, seq0 - 1, n_tok, st);
             else launch_prefill_hd<64, false>(p, seq0 - 1, n_tok, st);

@@ -705,33 +705,50 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillParams p) {
                                           pack2<RXQ4_DTYPE_F16>(acc[2] * inv, acc[3] * inv)};
 }
 
-// Launch model, microseconds, fitted to measured launches of 2 to 2048 tokens
-// after 0 to 16000 positions: a workgroup's fixed part and its tiles, the
-// workgroups' rounds over the CUs and, for splits, the partials' way through
-// memory and the second launch.
+// Launch model, microseconds: a workgroup's fixed part and its tiles, the
+// workgroups' rounds over the CUs and, for splits, the second launch and the
+// partials' way through memory.  Two sets of constants.  kSplit picks the split; its
+// workgroups are slower than those of a launch alone, which keeps launches of
+// several rounds from being cut too finely (with the second set for both, int8 1050
+// tokens, 32 / 8 heads of 64: 28.4 -> 39.2 us, 775 of 16 / 4 heads of 80 19.2 ->
+// 22.8).  The other gives the plan's time, against the other kernels' in the
+// dispatch, fitted to launches of 2 to 1500 tokens after 0 to 1500 positions: model
+// and measured, 32 / 8 heads of 128, fp16, 200 tokens 11.3 / 10.9, 512 16.6 / 16.6,
+// 400 after 400 23.2 / 23.0, 45 after 400 13.0 / 13.1 (4 chunks), 45 after 700 14.1 /
+// 14.0 (6), 130 after 600 18.3 / 18.7 (3).
 struct Cost {
-    double fixed, tile;
+    double fixed, tile, second, partials;  // partials: bytes a microsecond
 };
-Cost block_cost(int hd_pad) {
-    if (hd_pad == 64) return {4.7, 0.93};
-    if (hd_pad == 96) return {5.5, 1.15};
-    if (hd_pad == 128) return {6.5, 1.3};
-    return {6.0, 4.3};
+Cost split_cost(int hd_pad) {
+    if (hd_pad == 64) return {4.7, 0.93, 3.0, 3.5e6};
+    if (hd_pad == 96) return {5.5, 1.15, 3.0, 3.5e6};
+    if (hd_pad == 128) return {6.5, 1.3, 3.0, 3.5e6};
+    return {6.0, 4.3, 3.0, 3.5e6};
+}
+Cost time_cost(int hd_pad, int kv_int8) {
+    if (hd_pad == 64) return {kv_int8 ? 5.3 : 4.3, kv_int8 ? 1.2 : 0.93, 2.4, 2.6e6};
+    if (hd_pad == 96) return {kv_int8 ? 5.6 : 4.8, kv_int8 ? 1.3 : 1.1, 2.4, 2.6e6};
+    if (hd_pad == 128) return {kv_int8 ? 6.8 : 6.0, kv_int8 ? 1.55 : 1.32, 2.4, 2.6e6};
+    return {kv_int8 ? 6.3 : 5.9, kv_int8 ? 4.5 : 4.3, 2.4, 2.6e6};
+}
+// `tiles` the longest workgroup's, `work` and `units` all workgroups' tiles and
+// number, `bytes` of partials (0: no split).
+double launch_us(const Cost &k, int tiles, double work, double units, double bytes, int cus) {
+    double us = k.fixed + k.tile * tiles;
+    if (units > cus) us = std::max(us, (k.tile * work + 0.5 * k.fixed * units) / cus) + 0.3 * us;
+    return bytes > 0 ? us + k.second + bytes / k.partials : us;
 }
 
-struct Plan {
-    int chunk_tiles, n_chunks;
-    double us;
-};
 // The cheapest chunk of KV tiles per workgroup (a multiple of the G wave
 // groups) under the model.
-Plan plan_prefill(int64_t rows, int group, int n_kv, int start, int n_tok, int hd_pad, int G, int cus,
-                  size_t room) {
+PrefillPlan plan_prefill(int64_t rows, int group, int n_kv, int start, int n_tok, int hd_pad, int G,
+                         int kv_int8, int cus, size_t room) {
     const int tiles = (start + n_tok + kTile - 1) / kTile;
     const int64_t blocks = (rows + kBlock - 1) / kBlock;
     const int64_t step = (blocks + 7) / 8;  // up to eight blocks stand for all
-    const Cost k = block_cost(hd_pad);
-    Plan best{tiles, 1, 0};
+    const Cost pick = split_cost(hd_pad), time = time_cost(hd_pad, kv_int8);
+    PrefillPlan best{tiles, 1, 0};
+    double best_pick = 0;
     int last = 0;
     const int most = tuning().attn_split ? std::min(kMaxChunks, tuning().attn_split) : kMaxChunks;
     // 1, 2, 3, 4, 5, 6, 7, 8, 10, 12, .. splits, an eighth apart: a host call's worth
@@ -751,10 +768,13 @@ Plan plan_prefill(int64_t rows, int group, int n_kv, int start, int n_tok, int h
         }
         work *= blocks / seen * n_kv;
         units *= blocks / seen * n_kv;
-        double us = k.fixed + k.tile * std::min(ct, tiles);
-        if (units > cus) us = std::max(us, (k.tile * work + 0.5 * k.fixed * units) / cus) + 0.3 * us;
-        if (n_c > 1) us += 3.0 + (double)rows * n_kv * n_c * (hd_pad + 2) * 8 / 3.5e6;
-        if (best.us == 0 || us < best.us) best = Plan{ct, n_c, us};
+        const double chunk = (double)rows * (hd_pad + 2) * 8;  // a chunk of every block, per KV head
+        const double us = launch_us(pick, std::min(ct, tiles), work, units, n_c > 1 ? chunk * n_kv * n_c : 0, cus);
+        if (best_pick == 0 || us < best_pick) {
+            best_pick = us;
+            best = PrefillPlan{ct, n_c, launch_us(time, std::min(ct, tiles), work, units,
+                                                  n_c > 1 ? chunk * units / blocks : 0, cus)};
+        }
     }
     return best;
 }
@@ -762,12 +782,10 @@ Plan plan_prefill(int64_t rows, int group, int n_kv, int start, int n_tok, int h
 constexpr int kBigDim = 128;  // larger heads: one wave group, 512 registers a wave
 
 template <int HD, bool I8>
-hipError_t launch_prefill_t(PrefillParams &p, hipStream_t st) {
+hipError_t launch_prefill_t(PrefillParams &p, PrefillPlan plan, hipStream_t st) {
     constexpr int G = HD > kBigDim ? 1 : 2;
-    const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
     const int64_t rows = (int64_t)p.n_tok * p.group;
     const int64_t blocks = (rows + kBlock - 1) / kBlock;
-    Plan plan = plan_prefill(rows, p.group, p.n_kv, p.start, p.n_tok, HD, G, cus, kWorkspaceBytes);
     const int64_t units0 = blocks * p.n_kv;
     if (plan.n_chunks > 1) {
         float *ws = nullptr;
@@ -775,7 +793,7 @@ hipError_t launch_prefill_t(PrefillParams &p, hipStream_t st) {
         const hipError_t e = Scratch{}.get(st, (size_t)slots * kBlock * (HD + 2) * 4, &ws);
         if (e != hipSuccess) {
             (void)hipGetLastError();  // no workspace: the unsplit plan needs none
-            plan = Plan{(p.start + p.n_tok + kTile - 1) / kTile, 1, 0};
+            plan = PrefillPlan{(p.start + p.n_tok + kTile - 1) / kTile, 1, 0};
         } else {
             p.part = reinterpret_cast<f32x4 *>(ws);
             p.stats = ws + slots * kBlock * HD;
@@ -805,28 +823,27 @@ hipError_t launch_prefill_t(PrefillParams &p, hipStream_t st) {
 }
 
 template <bool I8>
-hipError_t launch_prefill_i(PrefillParams &p, hipStream_t st) {
-    if (p.hd <= 64) return launch_prefill_t<64, I8>(p, st);
-    if (p.hd <= 96) return launch_prefill_t<96, I8>(p, st);
-    if (p.hd <= 128) return launch_prefill_t<128, I8>(p, st);
-    return launch_prefill_t<256, I8>(p, st);
+hipError_t launch_prefill_i(PrefillParams &p, const PrefillPlan &plan, hipStream_t st) {
+    if (p.hd <= 64) return launch_prefill_t<64, I8>(p, plan, st);
+    if (p.hd <= 96) return launch_prefill_t<96, I8>(p, plan, st);
+    if (p.hd <= 128) return launch_prefill_t<128, I8>(p, plan, st);
+    return launch_prefill_t<256, I8>(p, plan, st);
 }
 
 }  // namespace
 
-double prefill_attention_us(int n_heads, int n_kv, int head_dim, int n_tok, int start) {
+PrefillPlan plan_prefill_attention(int n_heads, int n_kv, int head_dim, int n_tok, int start, int kv_int8) {
     const int cus = device_info().cu_count > 0 ? device_info().cu_count : 256;
     const int group = n_heads / n_kv;
     const int pad = head_dim <= 64 ? 64 : head_dim <= 96 ? 96 : head_dim <= 128 ? 128 : 256;
-    return plan_prefill((int64_t)n_tok * group, group, n_kv, start, n_tok, pad, pad > kBigDim ? 1 : 2, cus,
-                        kWorkspaceBytes)
-        .us;
+    return plan_prefill((int64_t)n_tok * group, group, n_kv, start, n_tok, pad, pad > kBigDim ? 1 : 2,
+                        kv_int8, cus, kWorkspaceBytes);
 }
 
 hipError_t launch_prefill_attention(uint16_t *out, const uint16_t *q, const void *k, const void *v,
                                     const float *ks, const float *vs, int n_heads, int n_kv,
                                     int head_dim, int n_tok, int start, float scale, int kv_int8,
-                                    hipStream_t st) {
+                                    const PrefillPlan &plan, hipStream_t st) {
     PrefillParams p{};
     p.out = out;
     p.q = q;
@@ -847,7 +864,7 @@ hipError_t launch_prefill_attention(uint16_t *out, const uint16_t *q, const void
     if ((int64_t)n_tok * p.group > 0x7FFFFF00 || (int64_t)n_kv * head_dim * 2 * kTile > 0x7FFFFF00 ||
         (int64_t)start + n_tok > 0x7FFFFF00)
         return hipErrorInvalidValue;
-    return kv_int8 ? launch_prefill_i<true>(p, st) : launch_prefill_i<false>(p, st);
+    return kv_int8 ? launch_prefill_i<true>(p, plan, st) : launch_prefill_i<false>(p, plan, st);
 }
 
 }  // namespace rxq4

@@ -171,12 +171,16 @@ hipError_t launch_attention(uint16_t *out, const uint16_t *q, const void *k, con
 
 // The same for two or more tokens, 128 query rows a workgroup and the positions
 // split over workgroups where that pays: token t sees positions [0, start + t].
-// prefill_attention_us: its launch model's time (the dispatch's measure).
-double prefill_attention_us(int n_heads, int n_kv, int head_dim, int n_tok, int start);
+// The plan holds the split and its launch model's time, the dispatch's measure.
+struct PrefillPlan {
+    int chunk_tiles, n_chunks;
+    double us;
+};
+PrefillPlan plan_prefill_attention(int n_heads, int n_kv, int head_dim, int n_tok, int start, int kv_int8);
 hipError_t launch_prefill_attention(uint16_t *out, const uint16_t *q, const void *k, const void *v,
                                     const float *ks, const float *vs, int n_heads, int n_kv,
                                     int head_dim, int n_tok, int start, float scale, int kv_int8,
-                                    hipStream_t stream);
+                                    const PrefillPlan &plan, hipStream_t stream);
 
 // fp32 rows -> Q4_K blocks (min/max quantiser).
 hipError_t launch_quantize(uint8_t *dst, const float *src, int64_t n_blocks,

@@ -71,6 +71,11 @@ PREFILL = [
     (4, 2, 72, 65, 128, False), (4, 4, 40, 33, 300, False), (2, 2, 8, 17, 100, False),
     (8, 4, 256, 40, 900, False), (3, 1, 256, 90, 65, "scales"), (5, 1, 136, 31, 2000, False),
     (8, 1, 16, 3, 70, "plain"),
+    # the VALU kernel's side of its line and the other: 2, 4 and 7 heads a group
+    # (four workgroups' worth of heads past 128 dims), one round of workgroups and
+    # more, int8
+    (32, 8, 80, 16, 40, False), (32, 8, 80, 3, 200, False), (5, 1, 256, 68, 0, False), (5, 1, 256, 68, 200, False),
+    (4, 4, 96, 68, 0, "scales"), (4, 4, 96, 200, 0, False), (14, 2, 160, 9, 60, "scales"), (4, 2, 72, 129, 0, False),
 ]
 
 
@@ -194,7 +199,7 @@ def test_prefill_attention_v_scales(H, KV, D, N, start, size):
 
 
 @pytest.mark.parametrize("what", ["nan", "inf", "-inf", "k", "scale", "k scale"])
-@pytest.mark.parametrize("H,KV,D,N,start", DIMS + [(2, 2, 80, 64, 64), (5, 1, 144, 31, 0), (4, 4, 48, 300, 1),
+@pytest.mark.parametrize("H,KV,D,N,start", DIMS + [(2, 2, 80, 64, 500), (8, 1, 144, 200, 0), (4, 4, 48, 300, 1),
                                                   (32, 8, 128, 45, 8000)])
 def test_prefill_attention_is_causal(H, KV, D, N, start, what):
     """Infinities and NaN in the caches reach the tokens that see them and no
