@@ -53,11 +53,12 @@
 // prefill_combine_kernel adds the chunks in order; plan_prefill picks the
 // chunk.
 //
-// Measured, 32 / 8 heads of 128, fp16 cache, against the 16-row kernel of
-// attn.hip (never split; graph replay): 45 tokens after 8000 positions 134 ->
-// 27 us, 128 after 16000 249 -> 69, 1000 from 0 35 -> 30, 2048 from 0 104 ->
-// 68, 4096 from 0 349 -> 230 (600 TFLOP/s); head_dim 80 and 256, which ran on
-// the VALU, 512 tokens 121 -> 16 and 185 -> 35 us.  Timing-only variants of an
+// Measured, 32 / 8 heads of 128, fp16 cache, other inputs each call, against the
+// 16-row kernel of attn.hip (never split): 45 tokens after 8000 positions 125.5 ->
+// 22.6 us, 128 after 16000 247 -> 61.5, 1000 from 0 31.4 -> 27.1, 2048 from 0 99.3 ->
+// 60.8, 4096 from 0 337 -> 216 (636 TFLOP/s); int8 2048 from 0 141 -> 69.4; head_dim
+// 80 and 256 against the VALU kernel, 512 tokens 115 -> 13.5 and 269 -> 39.7.
+// Timing-only variants (replays of one input, which run up to a fifth longer) of an
 // unsplit 8000-position walk (2.6 us per two tiles): without the tile loads
 // 2.3, without the exponentials 2.5, without P.V 1.8, without the low half of
 // P 2.2 us.  Not kept: half tiles of 32 positions with the next half's scores
@@ -338,7 +339,7 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_kernel(PrefillParams p) 
     // hold such positions those V values (int8: V scales) are staged again as
     // zeros, and the rows that see them get them at the end.  (Looked over after
     // their LDS writes have gone out: 300 tokens after 700 at head_dim 96 15.5 ->
-    // 15.8 us, 2048 from 0 at 128 unchanged; rows of a clean cache bit for bit.)
+    // 15.7 us, 2048 from 0 at 128 60.4 -> 60.9; rows of a clean cache bit for bit.)
     if (lane == 0) bad_v[w] = 0;  // the wave's flag: some of its staging
     auto look_over = [&](Raw &R, int t, int off, int s_off) {
         if (t * kTile + kTile - 1 <= blk_first) return;  // uniform
@@ -348,8 +349,11 @@ __global__ __launch_bounds__(256 * G) void attn_prefill_kernel(PrefillParams p) 
             if (bad && tid < kTile) scl[s_off + tid] = 0.0f;
         } else {
             if (__builtin_amdgcn_ballot_w64(not_finite16<NC>(R.c)) == 0) return;
-            zero_not_finite16<NC>(R.c);
-            store_raw(R, off, chunk_v, s_off);
+            Raw Z = R;  // (copies: head_dim 80, 775 tokens, 20.2 us with the loaded registers changed in place, 19.5)
+#pragma unroll
+            for (int j = 0; j < NC; ++j) asm volatile("" : "+v"(Z.c[j]));
+            zero_not_finite16<NC>(Z.c);
+            store_raw(Z, off, chunk_v, s_off);
         }
         if (lane == 0) bad_v[w] = 1;
     };
