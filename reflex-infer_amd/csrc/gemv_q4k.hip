@@ -21,6 +21,7 @@
 // Work: ~1.6 VALU ops per weight, under the ~2.8 ops/weight that 8 TB/s of
 // 4.5-bit weights leaves on 256 CUs.  Bytes per launch: rows*K/256*144 +
 // K*2 + rows*out_bytes (+ rows*2 residual).
+#include "gemv_units.h"
 #include "launch.h"
 #include "q4k_device.h"
 #include "rxq4.h"
@@ -243,7 +244,7 @@ __device__ __forceinline__ Range range_of_unit(const GemvParams &p, int unit) {
     const uint16_t *r0 = p.r[0].res, *r1 = p.r[1].res, *r2 = p.r[2].res;
     const int m0 = p.r[0].rows, m1 = p.r[1].rows, m2 = p.r[2].rows;
     const int u1 = p.unit_start[1], u2 = p.unit_start[2];
-    const int ri = (p.n_ranges > 1 && unit >= u1) ? ((p.n_ranges > 2 && unit >= u2) ? 2 : 1) : 0;
+    const int ri = range_index(unit, p.n_ranges, u1, u2);
     Range r;
     r.w = ri == 0 ? w0 : (ri == 1 ? w1 : w2);
     r.y = ri == 0 ? y0 : (ri == 1 ? y1 : y2);
@@ -697,8 +698,8 @@ __global__ __launch_bounds__(256) void gemv_lds_kernel(GemvParams p) {
     const Range rg = range_of_unit(p, active ? wave : 0);
     // inactive waves (the last workgroup's, when the units are not a multiple
     // of four) take no rows of range 0: their clamped loads read its row 0
-    const int r0 = active ? (wave - rg.first_unit) * p.per_unit : 0;
-    const int r1 = active ? min(r0 + p.per_unit, rg.rows) : 0;
+    const UnitSpan span = unit_span(active, wave, rg.first_unit, p.per_unit, rg.rows);
+    const int r0 = span.begin, r1 = span.end;
     const int n_items = (r1 - r0) * J;
     const uint32_t row_bytes = (uint32_t)p.nb * kBlockBytes;
 
@@ -711,7 +712,7 @@ __global__ __launch_bounds__(256) void gemv_lds_kernel(GemvParams p) {
     auto load = [&](Batch<U> &bt) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int row = max(0, min(ld_row, r1 - 1));
+            const int row = load_item(ld_row, r1);
             const int slot = min(64 * ld_j + lane, n_slots - 1);
             const uint8_t *blk = rg.w + (int64_t)row * row_bytes + (slot >> 2) * kBlockBytes;
             bt.h[u] = load16(blk);
@@ -1011,8 +1012,8 @@ __global__ __launch_bounds__(256) void gemv_rows_kernel(GemvParams p) {
     const bool active = wave < p.total_units;
     const Range rg = range_of_unit(p, active ? wave : 0);
     const int n_groups = (rg.rows + RPG - 1) / RPG;
-    const int g0 = active ? (wave - rg.first_unit) * p.per_unit : 0;
-    const int g1 = active ? min(g0 + p.per_unit, n_groups) : 0;
+    const UnitSpan span = unit_span(active, wave, rg.first_unit, p.per_unit, n_groups);
+    const int g0 = span.begin, g1 = span.end;
     const int n_items = (g1 - g0) * J;
     const uint32_t row_bytes = (uint32_t)p.nb * kBlockBytes;
     const int last = rg.rows - 1;
@@ -1021,7 +1022,7 @@ __global__ __launch_bounds__(256) void gemv_rows_kernel(GemvParams p) {
     // the range re-read its last row, steps past the wave's last group repeat
     // that group: loads are unconditional and in the range, results discarded.
     int ld_g = g0, ld_j = 0;
-    auto row_of = [&](int g) { return min(max(0, min(g, g1 - 1)) * RPG + sub, last); };
+    auto row_of = [&](int g) { return load_row(g, g1, RPG, sub, last); };
     const uint8_t *ld_row = rg.w + (int64_t)row_of(g0) * row_bytes;
     auto load = [&](Batch<U> &bt) {
 #pragma unroll
@@ -1175,17 +1176,11 @@ const DeviceInfo &device_info() {
 // Cut each range into units of `per_unit` items (an item is `rows_per_item`
 // rows); returns the unit count.  Units never straddle two ranges.
 static int assign_units(GemvParams &p, int rows_per_item, int per_unit) {
-    int units = 0;
-    p.unit_start[0] = 0;
-    for (int i = 0; i < p.n_ranges; ++i) {
-        if (i > 0) p.unit_start[i] = units;
-        const int items = (p.r[i].rows + rows_per_item - 1) / rows_per_item;
-        units += (items + per_unit - 1) / per_unit;
-    }
-    for (int i = p.n_ranges; i < 3; ++i) p.unit_start[i] = units;
+    int rows[3] = {};
+    for (int i = 0; i < p.n_ranges; ++i) rows[i] = p.r[i].rows;
     p.per_unit = per_unit;
-    p.total_units = units;
-    return units;
+    p.total_units = cut_units(rows, p.n_ranges, rows_per_item, per_unit, p.unit_start);
+    return p.total_units;
 }
 
 // Steps per load batch of the register kernel (two batches are in flight).

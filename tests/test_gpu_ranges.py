@@ -28,7 +28,8 @@ def host16(t: torch.Tensor) -> np.ndarray:
 # ------------------------------------------------- long rows, idle last waves
 # Rows of more than 64 slots whose waves hold more than 16 KB: the rows of the
 # ranges give 1022, 1021 and 1022 waves, so the last workgroup of four has
-# waves without rows (they must not read past range 0).
+# waves without rows.  (Parity: what those waves load is discarded; that it lies
+# in range 0 is tests/test_gemv_units.py's, on the CPU.)
 @pytest.mark.parametrize("rows,K", [((2503, 2604), 13824), ((5101,), 13824), ((1, 5099, 3), 13824)])
 def test_long_rows_with_idle_waves(rows, K):
     x = util.x_f16(7001, K)
