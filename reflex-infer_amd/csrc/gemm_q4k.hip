@@ -1352,7 +1352,12 @@ static hipError_t launch_tokens_t(void *y, const uint8_t *w, const uint16_t *x, 
     }
     // Short rows (nb < 16): the register kernel, never split over K (every
     // row is at most 15 super-blocks, dealt to the waves of one workgroup).
-    if (t2 * kWaves >= 1024 && wide) {  // (more tokens on as many rows: staged above)
+    // Two row tiles a workgroup where that still gives every CU one, up to 8
+    // tokens and half a 64-row workgroup per CU (past both x is staged above): on
+    // 256 CUs the 8192 rows of many models' layers.  [8192 x 2048] at 8 tokens 6.1 us,
+    // with one row tile 6.6, staged 7.4; gate, up and down of 8192 x 1024 at 8 16.1
+    // against 17.3 with one, 3584 24.7 against 27.2, 2048 at 4 18.0 against 17.9.
+    if (t2 >= cus && wide) {
         gemv_tokens_kernel<XT, YT, 2, kWaves, true><<<t2, kWaves * 64, 0, st>>>(y, w, x, M, n_tok, K);
         return hipGetLastError();
     }
