@@ -176,7 +176,11 @@ int rxq4_attention_decode_f16(void *out, const void *q, const void *k_cache,
  * hold past a token's last position does not reach its row, infinities and NaN
  * included, with one exception: at head_dim 64 and 128, where the launcher picks
  * the kernel for short prompts, an infinity or NaN in V or v_scales may reach
- * the earlier tokens of its 64-position tile.
+ * the earlier tokens of its 64-position tile.  Few tokens on long contexts split
+ * over the stream's workspace as decode does (without room for one the launch
+ * runs unsplit): a graph captured with such a call uses the capturing stream's,
+ * also where it is replayed on another, and must not be replayed once
+ * rxq4_release_workspace has freed it.
  * Replaces kernels::flash_attention_prefill_batched (reference
  * attention.cu:432-448, 180-290). */
 int rxq4_attention_prefill_f16(void *out, const void *q, const void *k_cache,

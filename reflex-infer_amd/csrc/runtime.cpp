@@ -1,8 +1,8 @@
 // runtime.cpp -- process-wide state of the library: the fp32 workspace of
 // the split launches and the tuning overrides read from the environment.
 //
-// Workspace (split-K GEMM partials, small-batch K-split partials,
-// decode-attention chunk partials):
+// Workspace (split-K GEMM partials, small-batch K-split partials of every
+// weight type, attention chunk partials of decode and prefill):
 // One buffer of kWorkspaceBytes per (device, stream), allocated the first
 // time a split launch is enqueued on that stream and kept until
 // rxq4_release_workspace frees it or the process ends.  Hence:

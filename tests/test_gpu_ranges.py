@@ -4,6 +4,10 @@ the CPU oracle (tests/util.py's tolerances) or a float64 product of the same
 operands."""
 from __future__ import annotations
 
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 import torch
@@ -265,6 +269,34 @@ def test_prefill_attention_split_in_a_graph():
         torch.cuda.synchronize()
         assert torch.equal(out, eager)
     capi.release_workspace(stream)
+
+
+def check_valu_attention():
+    """Every kernel of RXQ4_ATTN_MFMA=0, in a process of its own."""
+    g = torch.Generator(device="cuda").manual_seed(7250)
+    rnd = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    for H, KV, D, N, start, i8 in [(32, 8, 128, 45, 100, False), (7, 1, 64, 130, 0, True), (4, 4, 128, 3, 700, True),
+                                   (16, 1, 64, 20, 63, False), (8, 4, 256, 33, 200, False)]:
+        q, ks, vs = rnd(N, H * D).half(), None, None
+        if i8:
+            k, v = (rnd(start + N, KV, D).mul(40).round().clamp(-127, 127).to(torch.int8) for _ in range(2))
+            ks, vs = (rnd(start + N, KV).abs() * 0.01 + 0.005 for _ in range(2))
+        else:
+            k, v = rnd(start + N, KV, D).half(), rnd(start + N, KV, D).half()
+        out = torch.full((N, H * D), float("nan"), dtype=torch.float16, device="cuda")
+        capi.attention_prefill_f16(out, q, k, v, H, KV, D, N, start, D ** -0.5, i8, ks, vs)
+        ref = attention64(q, k, v, H, KV, D, N, start, D ** -0.5, ks, vs).cpu().numpy()
+        assert util.rounded_ok(host16(out).reshape(ref.shape), ref).all(), (H, KV, D, N, start, i8)
+
+
+def test_valu_attention_for_every_shape():
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    code = ("import sys; sys.path[:0] = [%r, %r]\nfrom tests import test_gpu_ranges as t\n"
+            "t.check_valu_attention()\nprint('valu ok')\n" % (root, os.path.join(root, "reflex-infer_amd")))
+    p = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, RXQ4_ATTN_MFMA="0"), capture_output=True,
+                       text=True, timeout=300)
+    assert p.returncode == 0, p.stderr[-2000:]
+    assert "valu ok" in p.stdout
 
 
 # ------------------------------------------------------- 17..64 token products
