@@ -1059,8 +1059,9 @@ static int valu_heads(int group, int head_dim) {
 // Other head sizes: the VALU kernel (a workgroup per token and head group), whose
 // tile costs by its heads.  Measured, this kernel / the other: 32 / 8 heads of 80, 3
 // tokens 4.9 / 6.0, 16 after 40 4.9 / 6.4, 3 after 200 12.1 / 8.7, 68 11.1 / 6.6; 4 / 4
-// heads of 96, 68 tokens 5.5 / 7.2, 3 after 200 7.6 / 8.5, 200 12.3 / 9.4; 5 / 1 heads
-// of 256, 16 after 40 6.4 / 10.3, 68 10.2 / 13.4, 68 after 200 19.6 / 13.7; int8 20
+// heads of 96, 68 tokens 5.5 / 7.2, 3 after 200 7.6 / 8.5, 200 12.3 / 9.4; 16 / 8 heads
+// of 80, 57 after 31 6.6 / 6.9, 100 10.0 / 6.8; 4 / 4, 128 5.6 / 7.4, 160 8.8 / 8.0; 5 / 1
+// heads of 256, 16 after 40 6.4 / 10.3, 68 10.2 / 13.4, 68 after 200 19.6 / 13.7; int8 20
 // after 100, 32 / 8 of 256, 12.2 / 13.9.
 static double valu_us(int n_heads, int n_kv, int head_dim, int n_tok, int start, int kv_int8, int cus) {
     const bool wide = head_dim > 128;
@@ -1070,9 +1071,11 @@ static double valu_us(int n_heads, int n_kv, int head_dim, int n_tok, int start,
     const double tile = kv_int8 ? 1.2 * per_tile : per_tile;
     const int tiles = (start + n_tok + kAttnTile - 1) / kAttnTile;
     const int64_t wgs = (int64_t)n_kv * ((group + hpw - 1) / hpw) * n_tok;
-    const int64_t rounds = (wgs + cus - 1) / cus;
-    const double one = (wide || hpw <= 2 ? 3.1 : 2.6) + tile * tiles;
-    return std::max(one, 2.0 + rounds * ((wide ? 2.0 : 0.8) + tile * mean_tiles(n_tok, start)));
+    // few heads of few dims leave registers for two workgroups a CU
+    const bool two = !wide && hpw <= 2;
+    const int64_t rounds = (wgs + (two ? 2 : 1) * cus - 1) / ((two ? 2 : 1) * cus);
+    const double one = (wide || two ? 3.1 : 2.6) + tile * tiles;
+    return std::max(one, 2.0 + rounds * ((wide ? 2.0 : two ? 1.5 : 0.8) + tile * mean_tiles(n_tok, start)));
 }
 
 template <int HD, bool I8>

@@ -80,7 +80,7 @@ PREFILL = [
     # (four workgroups' worth of heads past 128 dims), one round of workgroups and
     # more, int8
     (32, 8, 80, 16, 40, False), (32, 8, 80, 3, 200, False), (5, 1, 256, 68, 0, False), (5, 1, 256, 68, 200, False),
-    (4, 4, 96, 68, 0, "scales"), (4, 4, 96, 200, 0, False), (14, 2, 160, 9, 60, "scales"), (4, 2, 72, 129, 0, False),
+    (4, 4, 96, 68, 0, "scales"), (4, 4, 96, 200, 0, False), (4, 4, 80, 128, 0, False), (16, 8, 80, 57, 31, "scales"), (14, 2, 160, 9, 60, "scales"), (4, 2, 72, 129, 0, False),
 ]
 
 
